@@ -31,6 +31,9 @@ SIGNATURES = {
                   _i64, _i64, _f32, _vp], _i32),
     "vq2_gemv_rht": ([_vp, _i32, _i64, _i64, _vp, _vp, _i64, _f32, _i32, _vp, _i32, _vp, _vp, _i32, _i32, _i32,
                       _i64, _f32, _vp], _i32),
+    "vq2_rows_gemm_workspace": ([_i64, _i64, _i32, _vp, _i32, _i32], ctypes.c_size_t),
+    "vq2_rows_gemm": ([_vp, _i32, _i64, _i64, _vp, _vp, _i64, _f32, _i32, _i32, _vp, _i32, _vp, _vp, _i32, _i32, _i32,
+                       _i64, _f32, _vp, ctypes.c_size_t, _vp], _i32),
     "vq2_moe_gate_up_rht": ([_vp, _i32, _i64, _vp, _vp, _i64, _f32, _vp, _i32, _i64, _vp, _i64, _vp, _i32, _vp,
                              _i32, _vp, _i32, _i64, _i64, _i64, _f32, _vp], _i32),
     "vq2_moe_router_gate_up_rht": ([_vp, _i32, _i64, _vp, _vp, _i64, _f32, _vp, _i32, _i64, _i32, _vp, _i32, _i64,

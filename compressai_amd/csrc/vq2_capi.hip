@@ -289,6 +289,69 @@ int vq2_gemv_rht(const void* x, int x_dt, int64_t batch, int64_t x_stride, const
     return gemv_launch(c);
 }
 
+size_t vq2_rows_gemm_workspace(int64_t batch, int64_t n, int n_seg, const vq2_seg* segs, int s2_kind, int cb_dt)
+{
+    if (n_seg < 1 || n_seg > 4 || !segs) return 0;
+    RowsCall c{};
+    c.m = batch;
+    c.n = n;
+    c.s2 = s2_kind;
+    c.cb_dt = cb_dt;
+    c.nseg = n_seg;
+    for (int s = 0; s < n_seg; s++) c.seg[s].rows = segs[s].out_rows;
+    return rows_workspace_bytes(c);
+}
+
+int vq2_rows_gemm(const void* x, int x_dt, int64_t batch, int64_t x_stride, const int32_t* perm, const int8_t* sign,
+                  int64_t hb, float rht_scale, int act_dt, int n_seg, const vq2_seg* segs, int s2_kind,
+                  const void* cb0, const void* cb1, int cb_dt, int s_dt, int y_dt, int64_t n, float rs,
+                  void* workspace, size_t ws_bytes, void* stream)
+{
+    clear_error();
+    CHECK(batch >= 0 && n > 0 && n % 64 == 0, "vq2_rows_gemm: bad sizes batch=%lld n=%lld (a multiple of 64)",
+          (long long)batch, (long long)n);
+    CHECK(n_seg >= 1 && n_seg <= 4 && segs, "vq2_rows_gemm: 1..4 segments required");
+    if (batch == 0) return VQ2_OK;
+    CHECK(x, "vq2_rows_gemm: NULL activation");
+    CHECK(dt_ok(x_dt) && dt_ok(act_dt) && dt_ok(s_dt) && dt_ok(y_dt), "vq2_rows_gemm: bad dtype code");
+    CHECK(x_stride >= n, "vq2_rows_gemm: x_stride < n");
+    if (hb)
+        if (int rr = check_rot_tables(perm, sign)) return rr;
+    int r = check_codebooks(s2_kind, cb0, cb1, cb_dt);
+    if (r) return r;
+    RowsCall c{};
+    for (int s = 0; s < n_seg; s++) {
+        const vq2_seg& g = segs[s];
+        CHECK(g.out_rows >= 0, "vq2_rows_gemm: segment %d has negative rows", s);
+        CHECK(g.out_rows == 0 || (g.idx0 && g.scale && g.y), "vq2_rows_gemm: segment %d has a NULL pointer", s);
+        CHECK((s2_kind == VQ2_S2_NONE) == (g.idx1 == nullptr), "vq2_rows_gemm: segment %d idx1 mismatch", s);
+        CHECK(g.y_stride >= g.out_rows, "vq2_rows_gemm: segment %d y_stride < out_rows", s);
+        c.seg[s] = RowsSegCall{g.idx0, g.idx1, g.scale, g.y, g.out_rows, g.y_stride};
+    }
+    c.x = x;
+    c.x_dt = x_dt;
+    c.x_stride = x_stride;
+    c.m = batch;
+    c.perm = perm;
+    c.sign = sign;
+    c.hb = hb;
+    c.xscale = hb ? rht_scale : 1.0f;
+    c.act_dt = act_dt;
+    c.s2 = s2_kind;
+    c.cb0 = cb0;
+    c.cb1 = cb1;
+    c.cb_dt = cb_dt;
+    c.s_dt = s_dt;
+    c.y_dt = y_dt;
+    c.n = n;
+    c.rs = rs;
+    c.nseg = n_seg;
+    c.workspace = workspace;
+    c.ws_bytes = ws_bytes;
+    c.stream = stream;
+    return rows_launch(c);
+}
+
 int vq2_moe_grouped(const void* x, int x_dt, int64_t x_pair_stride, int64_t pairs_per_x, const void* ids,
                     int ids_dt, int64_t n_pairs, const int16_t* pool, int64_t n_experts, const void* cb, int cb_dt,
                     const void* pool_scale, int s_dt, void* y, int y_dt, int64_t y_pair_stride, int64_t out_rows,

@@ -119,6 +119,44 @@ int gemm_small_m_noalloc_launch(GemmCall c);
 size_t gemm_small_m_top1_workspace_bytes(int64_t m, int64_t out_rows, int64_t ng);
 int gemm_small_m_top1_launch(const GemmCall& c, int64_t* out_idx, float* out_val);
 
+// Rotation and matrix-core product of several rows (vq2_rows.hip).
+struct RowsSegCall {
+    const int16_t* idx0;
+    const void* idx1;
+    const void* scale;
+    void* y;
+    int64_t rows;
+    int64_t y_stride;  // elements between activation rows of y
+};
+
+struct RowsCall {
+    const void* x;
+    int x_dt;
+    int64_t x_stride;
+    int64_t m;
+    const int32_t* perm;
+    const int8_t* sign;
+    int64_t hb;  // 0: x is rotated
+    float xscale;
+    int act_dt;  // type the rotated activation is rounded to before fp16
+    int s2;
+    const void* cb0;
+    const void* cb1;
+    int cb_dt;
+    int s_dt;
+    int y_dt;
+    int64_t n;
+    float rs;
+    int nseg;
+    RowsSegCall seg[4];
+    void* workspace;
+    size_t ws_bytes;
+    void* stream;
+};
+
+size_t rows_workspace_bytes(const RowsCall& c);  // 0 for sizes that rows_launch refuses
+int rows_launch(const RowsCall& c);
+
 // VQ GEMV over the code-sorted internal layout (vq2_sorted.hip).
 struct SortedSegCall {
     const uint32_t* entries;   // [n_iters * 192] (768 bytes per iteration), 16-byte aligned

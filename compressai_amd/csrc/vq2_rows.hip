@@ -1,0 +1,669 @@
+// vq2_rows.hip -- several activation rows times up to 4 VQ matrices on the
+// gfx950 matrix cores, the rotation included.
+//
+//   y_s[m, r] = (sum_k RHT(x)[m, k] * W_s[r, k]) * scale_s[r] * rs,
+//   W[r, 8g + j] = cb0[i0[r, g]][j] (+ cb1[i1[r, g]][j]).
+//
+// Two launches for any number of rows:
+//  1. rows_pack_kernel: one workgroup per activation row rotates it (or takes
+//     it rotated), finds the row's power-of-two scale and writes it as fp16
+//     in the order the second launch's matrix instructions read (below).
+//     Codebooks that are not fp16 are rounded to fp16 by further workgroups
+//     of the same launch, so the second launch gathers 16 bytes a code.
+//  2. rows_gemm_kernel: the product.
+//
+// Why two launches and this layout.  The products are bound by the random
+// 16-byte centroid gathers, which the L2s serve at ~240 G/s whatever else the
+// chip does (bench_gather.hip), so a code must be gathered as few times as
+// possible, by a kernel with nothing else on its way.  A workgroup that
+// stages and converts its own activation (vq2_gemm_mfma.hip) does so once
+// per 64 output rows and K split and needs a third launch for the splits'
+// sum; here the activation is converted once, a wave reads its operand
+// fragments as whole 1 KiB lines straight into registers, and the K split
+// lies inside the workgroup (waves take k tiles in turn and their sums meet
+// in LDS), so nothing is written but y.  Measured (graph replays, us a call,
+// rotation included; before: vq2_rht, vq2_gemm_small_m per 64 rows and its
+// reduce launch): 2048 x 6144 at 4 bpw, 16 rows 29.3 -> 27.5; 6144 x 2048 at
+// 4 bpw, 64 rows 37.1 -> 31.2; two 6144 x 2048 at 3 bpw, 64 rows, bf16
+// 64.2 -> 38.6; 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5, 1024 rows
+// 264.8 -> 73.8.  Bound by the gathers (13 us of the 4 bpw calls) and, below
+// about a million codes, by the two launches' latency (~12 us).
+//
+// Fragment layout: v_mfma_f32_16x16x32_f16 takes 8 consecutive k of row
+// l % 16 from lane l, k block l / 16.  A k tile is 32 groups (256 k); its
+// step t (0..7) multiplies the groups 8q + t, q = 0..3, so that a lane's 8
+// codes of one matrix row and k tile are one 16-byte index load and step t's
+// gather is that lane's B operand as it arrives.  The packed activation holds,
+// for 16-row tile mt, k tile kt and step t, the 64 lanes' 16-byte operands in
+// lane order: chunk (((mt * KT + kt) * 8 + t) * 64 + q * 16 + row % 16).
+//
+// Precision: as vq2_gemm_mfma.hip: the rotation in fp32, one rounding to fp16
+// under a power-of-two scale per row (divided out of the fp32 sum exactly),
+// fp16 centroids as they are, fp32 accumulation.
+//
+// Semantics: the PackedLinear fallback for batch > 1, rotate, dequantize,
+// F.linear (vq2/runtime.py:82-89, 105-110), for (16,), (16,8) and (16,16).
+#include <algorithm>
+#include <mutex>
+
+#include "vq2_common.hpp"
+#include "vq2_internal.hpp"
+
+namespace vq2 {
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+constexpr int RW_TILE_G = 32;      // groups per k tile
+constexpr int RW_PACK_MAX = 1024;  // threads of a packing workgroup: one per group of its row
+constexpr int64_t RW_MAX_N = 8 * RW_PACK_MAX;
+constexpr int RW_CB_ROWS = 65536;
+
+// ------------------------------------------------------------- the packing
+struct RowsPackArgs {
+    const void* x;
+    int x_dt;
+    int x_vec;  // rows are 16-byte aligned
+    int64_t x_stride;
+    int64_t m;
+    int n;
+    int kt;       // k tiles
+    int hb_log2;  // 0: x is rotated
+    const int32_t* perm;
+    const int8_t* sign;
+    float scale;
+    int act_dt;  // type the rotated activation is rounded to first
+    half8_t* a;  // packed activation
+    int* e;      // exponent of each row's scale
+    uint32_t* cnt;  // arrival counters of the product, to be cleared
+    int n_cnt;
+    // codebooks to round to fp16 (null: none)
+    const void* cb0;
+    const void* cb1;
+    int cb_dt;
+    int cb1_rows;
+    half8_t* h0;
+    half8_t* h1;
+};
+
+__device__ __forceinline__ float rows_round_act(float v, int dt)
+{
+    if (dt == VQ2_DT_F16) return (float)(_Float16)v;
+    if (dt == VQ2_DT_BF16) return bf16_bits_to_f32(f32_to_bf16_bits(v));
+    return v;
+}
+
+// Centroid i of cb0, then cb1, rounded to fp16.
+__device__ __forceinline__ void rows_cvt_codebook(const RowsPackArgs& a, int64_t i)
+{
+    const void* src = a.cb0;
+    half8_t* dst = a.h0;
+    if (i >= RW_CB_ROWS) {
+        i -= RW_CB_ROWS;
+        src = a.cb1;
+        dst = a.h1;
+        if (i >= a.cb1_rows) return;
+    }
+    half8_t h;
+    if (a.cb_dt == VQ2_DT_BF16) {
+        const u32x4 u = *((const u32x4*)src + i);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            h[2 * k] = (_Float16)__uint_as_float(u[k] << 16);
+            h[2 * k + 1] = (_Float16)__uint_as_float(u[k] & 0xFFFF0000u);
+        }
+    } else {
+        const u32x4 lo = *((const u32x4*)src + 2 * i), hi = *((const u32x4*)src + 2 * i + 1);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            h[k] = (_Float16)__uint_as_float(lo[k]);
+            h[4 + k] = (_Float16)__uint_as_float(hi[k]);
+        }
+    }
+    dst[i] = h;
+}
+
+// Workgroup b < m: row b.  Thread t holds the 8 values of group t: value bits
+// 0-2 are in its registers, bits 3-8 across the lanes of its wave, 9-10 and
+// 11-12 across waves (one radix-4 exchange through LDS each).  The stages run
+// from bit 0 up, as in rht_kernel.  One group a thread keeps a 6144-value row
+// as fast as a 2048-value one: with 256 threads and three groups each it took
+// twice as long (11.4 against 5.8 us), serial latency on one wave per SIMD.
+__global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackArgs a)
+{
+    extern __shared__ __align__(16) float s_x[];  // the row; later the exchanges
+    __shared__ float s_max[RW_PACK_MAX / 64];
+    const int T = (int)blockDim.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t row = blockIdx.x;
+    if (row >= a.m) {
+        rows_cvt_codebook(a, (row - a.m) * T + tid);
+        return;
+    }
+    // the product's arrival counters
+    if (row == 0)
+        for (int i = tid; i < a.n_cnt; i += T) a.cnt[i] = 0u;
+    const int ng = a.n / 8;
+    const bool rot = a.hb_log2 > 0;
+    const bool g_ok = tid < ng;
+
+    // this thread's permutation and sign words, then the row into LDS
+    int32_t pw[8];
+    uint32_t sg[2];
+    if (rot) {
+        const int gc = g_ok ? tid : 0;
+        if (a.perm) {
+            const u32x4 p0 = *((const u32x4*)a.perm + 2 * gc), p1 = *((const u32x4*)a.perm + 2 * gc + 1);
+#pragma unroll
+            for (int k = 0; k < 4; k++) { pw[k] = (int32_t)p0[k]; pw[4 + k] = (int32_t)p1[k]; }
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; k++) pw[k] = gc * 8 + k;
+        }
+        if (a.sign) {
+            const u32x2 w = *((const u32x2*)a.sign + gc);
+            sg[0] = w.x;
+            sg[1] = w.y;
+        } else {
+            sg[0] = sg[1] = 0x01010101u;
+        }
+    }
+    const int64_t x0 = row * a.x_stride;
+    if (a.x_vec) {
+        if (a.x_dt == VQ2_DT_F32) {
+            const u32x4* xr = (const u32x4*)((const float*)a.x + x0);
+            for (int c = tid; c < a.n / 4; c += T) *((u32x4*)s_x + c) = xr[c];
+        } else if (g_ok) {
+            const u32x4 w = *((const u32x4*)((const uint16_t*)a.x + x0) + tid);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                s_x[tid * 8 + 2 * k] = a.x_dt == VQ2_DT_BF16 ? __uint_as_float(w[k] << 16)
+                                                             : f16_bits_to_f32((uint16_t)(w[k] & 0xFFFFu));
+                s_x[tid * 8 + 2 * k + 1] = a.x_dt == VQ2_DT_BF16 ? __uint_as_float(w[k] & 0xFFFF0000u)
+                                                                 : f16_bits_to_f32((uint16_t)(w[k] >> 16));
+            }
+        }
+    } else {
+        for (int i = tid; i < a.n; i += T) s_x[i] = load_as_f32(a.x, a.x_dt, x0 + i);
+    }
+    __syncthreads();
+
+    float v[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        if (!g_ok) {
+            v[k] = 0.0f;
+        } else if (!rot) {
+            v[k] = s_x[tid * 8 + k];
+        } else {
+            const bool bad = (uint32_t)pw[k] >= (uint32_t)a.n;  // not a permutation: poison, in bounds
+            const float s = (float)(int8_t)(sg[k >> 2] >> (8 * (k & 3)));
+            v[k] = bad ? __builtin_nanf("") : s_x[bad ? 0 : pw[k]] * s;
+        }
+    }
+    if (rot) {
+#pragma unroll
+        for (int h = 1; h < 8; h <<= 1)
+#pragma unroll
+            for (int k = 0; k < 8; k++)
+                if ((k & h) == 0) {
+                    const float p = v[k], q = v[k | h];
+                    v[k] = p + q;
+                    v[k | h] = p - q;
+                }
+        auto stage = [&](int bit, auto partner) {
+            if (a.hb_log2 > bit) {
+                const bool up = (lane >> (bit - 3)) & 1;
+#pragma unroll
+                for (int k = 0; k < 8; k++) {
+                    const float o = partner(v[k]);
+                    v[k] = up ? o - v[k] : v[k] + o;
+                }
+            }
+        };
+        stage(3, [](float f) { return dpp_xor1(f); });
+        stage(4, [](float f) { return dpp_xor2(f); });
+        stage(5, [](float f) { return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(f), 0x101F)); });
+        stage(6, [](float f) { return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(f), 0x201F)); });
+        stage(7, [](float f) { return swz_xor16(f); });
+        stage(8, [](float f) { return xor32(f); });
+        // bits b and b + 1 across waves: component k of group t at k * T + t
+        for (int b = 9; b < a.hb_log2; b += 2) {
+            const int d = 1 << (b - 3);
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < 8; k++) s_x[k * T + tid] = v[k];
+            __syncthreads();
+            const bool u0 = tid & d, u1 = tid & (2 * d), two = a.hb_log2 > b + 1;
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                const float o = s_x[k * T + (tid ^ d)];
+                const float r = u0 ? o - v[k] : v[k] + o;
+                if (two) {
+                    const float p2 = s_x[k * T + (tid ^ (2 * d))], o2 = s_x[k * T + (tid ^ (3 * d))];
+                    const float r2 = u0 ? o2 - p2 : p2 + o2;
+                    v[k] = u1 ? r2 - r : r + r2;
+                } else {
+                    v[k] = r;
+                }
+            }
+        }
+    }
+    float am = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        if (rot) v[k] = rows_round_act(v[k] * a.scale, a.act_dt);
+        am = fmaxf(am, fabsf(v[k]));  // skips NaN, which reaches its output row through the product
+    }
+    am = wave_max_all(am);
+    if (lane == 0) s_max[wave] = am;
+    __syncthreads();
+    for (int w = 0; w < T / 64; w++) am = fmaxf(am, s_max[w]);
+    // the row's largest value into [2^14, 2^15): exact, far below 65504; a
+    // row of zeros or with an infinity keeps scale 1
+    const uint32_t ab = __float_as_uint(am);
+    const int e = ab != 0u && ab < 0x7F800000u ? 14 - ilogbf(am) : 0;
+    if (tid == 0) a.e[row] = e;
+    const int kt = tid / RW_TILE_G, t = tid & 7, q = (tid >> 3) & 3;
+    if (kt >= a.kt) return;
+    half8_t h;
+#pragma unroll
+    for (int k = 0; k < 8; k++) h[k] = (_Float16)ldexpf(v[k], e);
+    a.a[(((row >> 4) * a.kt + kt) * 8 + t) * 64 + q * 16 + (row & 15)] = h;
+}
+
+// ------------------------------------------------------------- the product
+struct RowsSeg {
+    const int16_t* idx0;
+    const void* idx1;
+    const void* scale;
+    void* y;
+    int64_t y_stride;
+    int rows;
+    int tile0;  // first column tile of this matrix
+};
+
+struct RowsArgs {
+    const half8_t* a;  // packed activation
+    const int* e;
+    int m;
+    int kt;  // k tiles
+    int ng;
+    const half8_t* cb0;  // fp16 codebooks
+    const half8_t* cb1;
+    int s_dt;
+    int y_dt;
+    float rs;
+    int nseg;
+    int kw;  // waves of a workgroup that share a column tile's k tiles
+    int nz;  // workgroups that share them (gridDim.z); nc is 1 then
+    float* part;    // nz > 1: [row block][column tile][nz][16 MT][16 NT] sums
+    uint32_t* cnt;  // nz > 1: arrivals per [row block][column tile], zero
+    RowsSeg seg[4];
+};
+
+// A wave's codes of one column (16 columns a wave, lane l: column l % 16)
+// and k tile: the 8 groups 8 (l / 16) + t.
+template <int S2>
+struct RowCodes {
+    u32x4 w0;
+    u32x4 w1;  // (16,8): the first two words
+    __device__ __forceinline__ void load(const RowsSeg& s, int64_t off)
+    {
+        w0 = __builtin_nontemporal_load((const u32x4*)(s.idx0 + off));
+        if constexpr (S2 == VQ2_S2_U16) w1 = __builtin_nontemporal_load((const u32x4*)((const int16_t*)s.idx1 + off));
+        if constexpr (S2 == VQ2_S2_U8) {
+            const u32x2 w = __builtin_nontemporal_load((const u32x2*)((const uint8_t*)s.idx1 + off));
+            w1[0] = w.x;
+            w1[1] = w.y;
+        }
+    }
+    __device__ __forceinline__ uint32_t c0(int t) const { return (w0[t >> 1] >> (16 * (t & 1))) & 0xFFFFu; }
+    __device__ __forceinline__ uint32_t c1(int t) const
+    {
+        if constexpr (S2 == VQ2_S2_U8) return (w1[t >> 2] >> (8 * (t & 3))) & 0xFFu;
+        else return (w1[t >> 1] >> (16 * (t & 1))) & 0xFFFFu;
+    }
+};
+
+__device__ __forceinline__ const RowsSeg& rows_seg(const RowsArgs& a, int tile)
+{
+    int s = 0;
+    for (int i = 1; i < a.nseg; i++) s += tile >= a.seg[i].tile0 ? 1 : 0;
+    return a.seg[s];
+}
+
+constexpr int RW_MAX_WAVES = 16;
+constexpr int RW_MAX_Z = 4;  // workgroups that share a tile's k tiles
+
+// Up to 16 * MT rows: a workgroup is nc column tiles of 16 * NT columns x kw
+// waves over the k tiles; blockIdx.y counts blocks of 16 * MT rows.
+template <int S2, int MT, int NT>
+__global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const RowsArgs a)
+{
+    touch_kernargs(a);
+    extern __shared__ __align__(16) float s_red[];  // [waves][16 MT][16 NT + 1]
+    __shared__ half8_t s_c1[S2 == VQ2_S2_U8 ? 256 : 1];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nl = lane & 15, q = lane >> 4;
+    const int kw = a.kw, nc = (int)(blockDim.x >> 6) / kw;
+    const int tile = (int)blockIdx.x * nc + wave / kw;
+    const int k0 = (int)blockIdx.z * kw + wave % kw, kstep = kw * a.nz;
+    const RowsSeg& sg = rows_seg(a, tile);
+    const int col0 = (tile - sg.tile0) * 16 * NT;  // may lie past the last matrix's rows (tail workgroup)
+    const int mt0 = (int)blockIdx.y * MT;
+    const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+
+    if constexpr (S2 == VQ2_S2_U8) {
+        for (int i = tid; i < 256; i += (int)blockDim.x) s_c1[i] = a.cb1[i];
+        __syncthreads();
+    }
+
+    int64_t rowoff[NT];
+#pragma unroll
+    for (int c = 0; c < NT; c++) {
+        const int r = col0 + c * 16 + nl;
+        rowoff[c] = (int64_t)(r < sg.rows ? r : 0) * a.ng;
+    }
+    // row tiles past the last one read tile mt_last again (results dropped)
+    const int mt_last = (a.m - 1) >> 4;
+    const half8_t* ap[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) ap[i] = a.a + (int64_t)min(mt0 + i, mt_last) * a.kt * 512 + lane;
+
+    f32x4_t acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int c = 0; c < NT; c++) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+
+    RowCodes<S2> cd[NT];
+    auto load_codes = [&](int kt) {
+        // the last k tile may be short: whole k blocks of 8 groups are missing
+        const int g = kt * RW_TILE_G + q * 8;
+#pragma unroll
+        for (int c = 0; c < NT; c++) cd[c].load(sg, rowoff[c] + (g < a.ng ? g : 0));
+    };
+    if (k0 < a.kt) load_codes(k0);
+    for (int kt = k0; kt < a.kt; kt += kstep) {
+        const bool g_ok = kt * RW_TILE_G + q * 8 < a.ng;
+        half8_t b0[8][NT], b1[8][NT];
+#pragma unroll
+        for (int t = 0; t < 8; t++)
+#pragma unroll
+            for (int c = 0; c < NT; c++) {
+                b0[t][c] = a.cb0[cd[c].c0(t)];
+                if constexpr (S2 == VQ2_S2_U16) b1[t][c] = a.cb1[cd[c].c1(t)];
+                if constexpr (S2 == VQ2_S2_U8) b1[t][c] = s_c1[cd[c].c1(t)];
+            }
+        if (kt + kstep < a.kt) load_codes(kt + kstep);
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            half8_t av[MT];
+#pragma unroll
+            for (int i = 0; i < MT; i++) av[i] = ap[i][((int64_t)kt * 8 + t) * 64];
+#pragma unroll
+            for (int c = 0; c < NT; c++) {
+                const half8_t bb = g_ok ? b0[t][c] : zero8;
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bb, acc[i][c], 0, 0, 0);
+                if constexpr (S2 != VQ2_S2_NONE) {
+                    const half8_t bc = g_ok ? b1[t][c] : zero8;
+#pragma unroll
+                    for (int i = 0; i < MT; i++)
+                        acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bc, acc[i][c], 0, 0, 0);
+                }
+            }
+        }
+    }
+
+    // D[i][j]: activation row 4 (l / 16) + e of the tile, column l % 16; the
+    // waves' sums meet in LDS and are added in wave order
+    constexpr int LD = 16 * NT + 1, TILE = 16 * MT * LD;
+    float* mine = s_red + wave * TILE;
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int c = 0; c < NT; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) mine[(i * 16 + q * 4 + e) * LD + c * 16 + nl] = acc[i][c][e];
+    __syncthreads();
+    const int mrows = min(16 * MT, a.m - mt0 * 16);
+    const float* red = s_red;
+    int nred = kw;
+    if (a.nz > 1) {
+        // this workgroup's sums; the last of the tile's workgroups adds them
+        // in order (arrive_last)
+        const int64_t unit = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+        float* pt = a.part + (unit * a.nz + blockIdx.z) * (256 * MT * NT);
+        for (int t = tid; t < 256 * MT * NT; t += (int)blockDim.x) {
+            const float* p = s_red + t / (16 * NT) * LD + t % (16 * NT);
+            float sum = 0.0f;
+            for (int w = 0; w < kw; w++) sum += p[w * TILE];
+            share_store(pt + t, sum);
+        }
+        if (!arrive_last(a.cnt + unit, (uint32_t)a.nz)) return;
+        pt = a.part + unit * a.nz * (256 * MT * NT);
+        for (int t = tid; t < 256 * MT * NT; t += (int)blockDim.x) {
+            // at most RW_MAX_Z partials, their loads in flight together
+            float v[RW_MAX_Z], sum = 0.0f;
+#pragma unroll
+            for (int z = 0; z < RW_MAX_Z; z++) v[z] = share_load(pt + min(z, a.nz - 1) * (256 * MT * NT) + t);
+#pragma unroll
+            for (int z = 0; z < RW_MAX_Z; z++) sum += z < a.nz ? v[z] : 0.0f;
+            s_red[t / (16 * NT) * LD + t % (16 * NT)] = sum;
+        }
+        __syncthreads();
+        nred = 1;
+    }
+    for (int t = tid; t < nc * mrows * 16 * NT; t += (int)blockDim.x) {
+        const int c = t % (16 * NT), u = t / (16 * NT);
+        const int r = u % mrows, ct = u / mrows;
+        const int tl = (int)blockIdx.x * nc + ct;
+        const RowsSeg& so = rows_seg(a, tl);
+        const int col = (tl - so.tile0) * 16 * NT + c;
+        if (col >= so.rows) continue;
+        const float* p = red + ct * kw * TILE + r * LD + c;
+        float sum = 0.0f;
+        for (int w = 0; w < nred; w++) sum += p[w * TILE];
+        const int row = mt0 * 16 + r;
+        const float s = load_as_f32(so.scale, a.s_dt, col);
+        store_from_f32(so.y, a.y_dt, (int64_t)row * so.y_stride + col, (ldexpf(sum, -a.e[row]) * s) * a.rs);
+    }
+}
+
+// ------------------------------------------------------------------ launch
+struct RowsPlan {
+    int kt;
+    int mt, nt;        // 16-row and 16-column tiles of a wave
+    int kw, nc, nz;    // waves and workgroups over a column tile's k tiles; column tiles of a workgroup
+    int64_t tiles;     // column tiles of all matrices
+    int64_t grid_x, grid_y;
+    // workspace: arrival counters, the rows' exponents, the packed
+    // activation, fp16 codebooks, the partial sums of nz > 1
+    size_t e, a, h0, h1, part, total;
+};
+
+static size_t up256(size_t b) { return (b + 255) / 256 * 256; }
+
+static RowsPlan rows_plan(const RowsCall& c)
+{
+    RowsPlan p{};
+    p.kt = (int)((c.n / 8 + RW_TILE_G - 1) / RW_TILE_G);
+    p.mt = (int)std::min<int64_t>(4, (c.m + 15) / 16);
+    p.nt = 1;
+    for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 16 * p.nt - 1) / (16 * p.nt);
+    p.grid_y = (c.m + 16 * p.mt - 1) / (16 * p.mt);
+    // Few column tiles leave CUs idle, and a CU gathers at most ~0.9 codes a
+    // ns however few others do: several workgroups then share a tile's k
+    // tiles, while a workgroup has 6144 gathers or more (below that the
+    // sum over workgroups costs more, ~1.5 us: 2048 x 2048 at 2 bpw, 16 rows,
+    // 4096 gathers 13.7 us a call, two workgroups 14.4; at 4 bpw 18.3 / 17.5;
+    // 2048 x 6144 at 4 bpw 34.5 / 28.3; 512 x 6144 40.1 / 26.3 / 20.7 with
+    // four) and the launch stays within a workgroup per CU.
+    const int64_t gathers = 16 * p.nt * (c.n / 8) * (c.s2 == VQ2_S2_U16 ? 2 : 1);
+    p.nz = 1;
+    while (2 * p.nz <= std::min(RW_MAX_Z, p.kt) && 2 * p.nz * p.tiles * p.grid_y <= device_cu_count() &&
+           gathers / p.nz >= 6144)
+        p.nz *= 2;
+    // the k tiles over up to 16 waves, as evenly as whole tiles allow; short
+    // reductions put several column tiles into a workgroup of 8 waves where
+    // every CU still has one (1024 x 1024 at 4 bpw in 32 workgroups of two
+    // tiles took 18.6 us a call, in 64 of one 13.9)
+    const int per = (p.kt + p.nz - 1) / p.nz, rounds = (per + RW_MAX_WAVES - 1) / RW_MAX_WAVES;
+    p.kw = (per + rounds - 1) / rounds;
+    p.nc = (int)std::max<int64_t>(1, std::min<int64_t>(8 / p.kw, p.tiles * p.grid_y / device_cu_count()));
+    p.grid_x = (p.tiles + p.nc - 1) / p.nc;
+    const bool cvt = c.cb_dt != VQ2_DT_F16;
+    const int64_t units = p.nz > 1 ? p.grid_x * p.grid_y : 0;
+    p.e = up256((size_t)units * sizeof(uint32_t));
+    p.a = p.e + up256((size_t)c.m * sizeof(int));
+    p.h0 = p.a + (size_t)((c.m + 15) / 16) * p.kt * 512 * sizeof(half8_t);
+    p.h1 = p.h0 + (cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
+    p.part = p.h1 + (!cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
+    p.total = p.part + (size_t)units * p.nz * 256 * p.mt * p.nt * sizeof(float);
+    return p;
+}
+
+static int rows_check(const RowsCall& c)
+{
+    if (c.n > RW_MAX_N || c.n < 64 || c.n % 64)
+        return set_error(VQ2_ERR_UNSUPPORTED, "vq2_rows_gemm: n=%lld must be a multiple of 64 up to %lld", (long long)c.n,
+                         (long long)RW_MAX_N);
+    if (c.m < 1 || c.m > 1 << 20)
+        return set_error(VQ2_ERR_UNSUPPORTED, "vq2_rows_gemm: %lld activation rows outside 1..2^20", (long long)c.m);
+    for (int s = 0; s < c.nseg; s++)
+        if (c.seg[s].rows < 0 || c.seg[s].rows > 0x0FFFFFFF)
+            return set_error(VQ2_ERR_UNSUPPORTED, "vq2_rows_gemm: matrix %d has %lld rows", s, (long long)c.seg[s].rows);
+    return VQ2_OK;
+}
+
+size_t rows_workspace_bytes(const RowsCall& c)
+{
+    return rows_check(c) == VQ2_OK ? rows_plan(c).total : 0;
+}
+
+template <int S2, int MT, int NT>
+static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
+{
+    // opt in to more than 64 KiB of dynamic LDS, once per instantiation
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    constexpr size_t SHM_WAVE = 16 * MT * (16 * NT + 1) * sizeof(float);
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT, NT>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RW_MAX_WAVES * SHM_WAVE));
+    });
+    if (attr != hipSuccess) return attr;
+    const size_t shm = waves * SHM_WAVE;
+    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT, NT>), grid, dim3(64 * waves), shm, st, a);
+    return hipGetLastError();
+}
+
+template <int S2>
+static hipError_t rows_launch_s(int mt, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
+{
+    switch (mt) {
+    case 1: return rows_launch_t<S2, 1, 1>(a, grid, waves, st);
+    case 2: return rows_launch_t<S2, 2, 1>(a, grid, waves, st);
+    case 3: return rows_launch_t<S2, 3, 1>(a, grid, waves, st);
+    default: return rows_launch_t<S2, 4, 1>(a, grid, waves, st);
+    }
+}
+
+static hipError_t rows_pack_launch(const RowsPackArgs& p, hipStream_t st)
+{
+    const int T = std::max(64, (p.kt * RW_TILE_G + 63) / 64 * 64);
+    int64_t blocks = p.m;
+    if (p.cb0) blocks += (RW_CB_ROWS + p.cb1_rows + T - 1) / T;
+    const size_t shm = (size_t)T * 8 * sizeof(float);
+    hipLaunchKernelGGL(rows_pack_kernel, dim3((unsigned)blocks), dim3(T), shm, st, p);
+    return hipGetLastError();
+}
+
+int rows_launch(const RowsCall& c)
+{
+    if (int r = rows_check(c)) return r;
+    int hl = 0;
+    while ((1LL << hl) < c.hb) hl++;
+    if (c.hb && ((1LL << hl) != c.hb || c.hb < 64 || c.n % c.hb))
+        return set_error(VQ2_ERR_ARG, "vq2_rows_gemm: hb=%lld must be 0 or a power of two of at least 64 dividing n",
+                         (long long)c.hb);
+    for (int s = 0; s < c.nseg; s++) {
+        const RowsSegCall& g = c.seg[s];
+        const uintptr_t al = (uintptr_t)g.idx0 | (c.s2 == VQ2_S2_U16 ? (uintptr_t)g.idx1 : 0);
+        if (al % 16 || (c.s2 == VQ2_S2_U8 && (uintptr_t)g.idx1 % 8))
+            return set_error(VQ2_ERR_UNSUPPORTED, "vq2_rows_gemm: index planes must be 16-byte aligned");
+    }
+    const RowsPlan p = rows_plan(c);
+    if (p.tiles == 0) return VQ2_OK;
+    if (p.grid_x > 0x3FFFFFFF || p.grid_y > 65535)
+        return set_error(VQ2_ERR_UNSUPPORTED, "vq2_rows_gemm: grid too large");
+    if (!c.workspace || c.ws_bytes < p.total || (uintptr_t)c.workspace % 256)
+        return set_error(VQ2_ERR_ARG, "vq2_rows_gemm: workspace of %zu bytes (256-byte aligned) needed, got %zu", p.total,
+                         c.ws_bytes);
+    char* ws = (char*)c.workspace;
+    const bool cvt = c.cb_dt != VQ2_DT_F16;
+    hipStream_t st = (hipStream_t)c.stream;
+
+    RowsPackArgs k{};
+    k.x = c.x;
+    k.x_dt = c.x_dt;
+    k.x_vec = (uintptr_t)c.x % 16 == 0 && (c.x_stride * dt_size(c.x_dt)) % 16 == 0;
+    k.x_stride = c.x_stride;
+    k.m = c.m;
+    k.n = (int)c.n;
+    k.kt = p.kt;
+    k.hb_log2 = c.hb ? hl : 0;
+    k.perm = c.perm;
+    k.sign = c.sign;
+    k.scale = c.xscale;
+    k.act_dt = c.act_dt;
+    k.a = (half8_t*)(ws + p.a);
+    k.e = (int*)(ws + p.e);
+    k.cnt = (uint32_t*)ws;
+    k.n_cnt = p.nz > 1 ? (int)(p.grid_x * p.grid_y) : 0;
+    if (cvt) {
+        k.cb0 = c.cb0;
+        k.cb1 = c.cb1;
+        k.cb_dt = c.cb_dt;
+        k.cb1_rows = c.s2 == VQ2_S2_NONE ? 0 : (c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS);
+        k.h0 = (half8_t*)(ws + p.h0);
+        k.h1 = (half8_t*)(ws + p.h1);
+    }
+    hipError_t err = rows_pack_launch(k, st);
+    if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm packing launch");
+
+    RowsArgs a{};
+    a.a = k.a;
+    a.e = k.e;
+    a.m = (int)c.m;
+    a.ng = (int)(c.n / 8);
+    a.kt = p.kt;
+    a.cb0 = cvt ? k.h0 : (const half8_t*)c.cb0;
+    a.cb1 = cvt ? k.h1 : (const half8_t*)c.cb1;
+    a.s_dt = c.s_dt;
+    a.y_dt = c.y_dt;
+    a.rs = c.rs;
+    a.kw = p.kw;
+    a.nz = p.nz;
+    a.part = (float*)(ws + p.part);
+    a.cnt = k.cnt;
+    int64_t tile = 0;
+    for (int s = 0; s < c.nseg; s++) {
+        const RowsSegCall& g = c.seg[s];
+        if (g.rows == 0) continue;
+        a.seg[a.nseg++] = RowsSeg{g.idx0, g.idx1, g.scale, g.y, g.y_stride, (int)g.rows, (int)tile};
+        tile += (g.rows + 16 * p.nt - 1) / (16 * p.nt);
+    }
+    const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y, (unsigned)p.nz);
+    switch (c.s2) {
+    case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, a, grid, p.kw * p.nc, st); break;
+    case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, a, grid, p.kw * p.nc, st); break;
+    default: err = rows_launch_s<VQ2_S2_NONE>(p.mt, a, grid, p.kw * p.nc, st); break;
+    }
+    if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm launch");
+    return VQ2_OK;
+}
+
+}  // namespace vq2

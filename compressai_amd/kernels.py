@@ -475,6 +475,46 @@ def vq_gemv_rht(x, mats, cb0, cb1, n, perm=None, sign=None, hb=2048, rht_scale=N
     return outs
 
 
+# Widest rows that vq_rows_gemm takes: its packing workgroup holds one row.
+ROWS_GEMM_MAX_N = 8192
+
+
+def vq_rows_gemm(x, mats, cb0, cb1, n, perm=None, sign=None, hb=2048, rht_scale=None, rs=1.0, *,
+                 act_dtype=torch.float32, out_dtype=torch.float32, ys=None):
+    """Rotate x [B, n] with the RHT (hb = 0: x is rotated) and multiply by up
+    to 4 VQ matrices on the matrix cores, for any B: two launches, the rotated
+    rows (rounded to act_dtype, then to fp16 under a power-of-two scale per
+    row) packed for the product.  n a multiple of 64 up to ROWS_GEMM_MAX_N;
+    mats: list of (i0, i1 or None, scale, out_rows) sharing one cfg.  Returns
+    the list of outputs [B, out_rows]."""
+    n = int(n)
+    s2, mats = check_gemv_rht_mats(mats, cb0, cb1, n)
+    dev = _dev(x, cb0, cb1, perm, sign, *[t for m in mats for t in m[:3]])
+    x2 = _contig(x, "x").reshape(-1, n)
+    B = x2.shape[0]
+    _perm_sign(perm, sign, n)
+    if n % 64 or n > ROWS_GEMM_MAX_N:
+        raise Vq2Error(f"vq_rows_gemm: n={n} must be a multiple of 64 up to {ROWS_GEMM_MAX_N}")
+    if act_dtype not in _DT:
+        raise Vq2Error(f"vq_rows_gemm: unsupported act_dtype {act_dtype}")
+    if ys is None:
+        ys = [torch.empty((B, m[3]), dtype=out_dtype, device=dev) for m in mats]
+    segs = (_lib.Seg * len(mats))()
+    for k, ((i0, i1, scale, out_rows), y) in enumerate(zip(mats, ys)):
+        _contig(y, "y")
+        if y.numel() != B * out_rows or y.dtype != ys[0].dtype or y.device != dev:
+            raise Vq2Error(f"vq_rows_gemm: output {k} must be [{B}, {out_rows}] of the launch's dtype on {dev}")
+        segs[k] = _lib.Seg(_p(i0), _p(i1), _p(scale), _p(y), out_rows, out_rows)
+    hb = int(hb or 0)
+    sc = (float(hb) ** -0.5 if hb else 1.0) if rht_scale is None else float(rht_scale)
+    cdt = _dt(cb0, "cb0")
+    ws = torch.empty(_lib.load().vq2_rows_gemm_workspace(B, n, len(mats), segs, s2, cdt), dtype=torch.uint8, device=dev)
+    _lib.call("vq2_rows_gemm", _p(x2), _dt(x2, "x"), B, n, _p(perm), _p(sign), hb, sc, _DT[act_dtype], len(mats), segs,
+              s2, _p(cb0), _p(cb1), cdt, _dt(mats[0][2], "scale"), _dt(ys[0], "y"), n, float(rs), _p(ws), ws.numel(),
+              _stream(dev))
+    return ys
+
+
 # ------------------------------------------------------- code-sorted layout
 # uint32 words per iteration of the sorted layout: 64 lanes x 12 bytes, the
 # four 64-lane instructions of 63 codes and one base code each

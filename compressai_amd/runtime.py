@@ -5,8 +5,8 @@ reference constructor (vq2/runtime.py:70-80): ``idx`` is the list of index
 planes (int16 for 16-bit stages, uint8 for 8-bit stages), ``scale`` the
 per-row scales, ``cbs`` a dict of codebooks keyed by the cfg prefix
 ("16", "16_8", "16_16").  ``forward(x)`` rotates x with the layer's RHT and
-runs the fused VQ GEMV (batch <= 2) or the matrix-core small-M GEMM
-(batch >= 3) for every cfg in (16,), (16, 8), (16, 16) -- the reference
+runs the fused VQ GEMV (batch <= 2) or the matrix-core product of all rows
+(batch >= 3, ``kernels.vq_rows_gemm``) for every cfg in (16,), (16, 8), (16, 16) -- the reference
 fuses only batch 1 of (16,) and (16, 8) and otherwise re-materialises the
 dequantized matrix (runtime.py:91-110).
 ``PackedLMHead`` (runtime.py:136-144) wraps it and adds ``argmax``.
@@ -31,7 +31,7 @@ def cfg_key(cfg, i):
     return "_".join(str(b) for b in cfg[: i + 1])
 
 
-# batch rows per matrix-core launch (vq2_gemm_small_m takes up to 64)
+# batch rows per launch of vq2_gemm_small_m (rows wider than vq_rows_gemm takes)
 SMALL_M_MAX = 64
 
 # matrices with at least this many codes (all stages) use the code-sorted
@@ -58,15 +58,15 @@ SORTED_MIN_LAUNCH_CODES = SORTED_MIN_CODES
 #    batch 4, top-1 or logits;
 #  * batch 2 of inputs wider than 2048 (down 2048 x 6144, 4 bpw: 22.4 against
 #    28.9 on the gather kernel with the 6144-point RHT in its prologue);
-#  * PackedProjections at batch 3-4 (q, k, v in one launch: 22.0-24.4 against
-#    35.9-36.1 for the three projections on the matrix cores; gate + up:
-#    40.1-42.0 against 47.0-47.4), and at batch 2 with
-#    SORTED_BATCH2_LAUNCH_MIN_CODES codes or more (gate + up: 24.6 against
-#    37.6 in one gather-kernel launch).
+#  * PackedProjections at batch 2 with SORTED_BATCH2_LAUNCH_MIN_CODES codes or
+#    more (gate + up: 24.6 against 37.6 in one gather-kernel launch).
 # Not used where it was slower: one 6144 x 2048 4 bpw matrix at batch 2
-# (23.2 against 20.9) and 3-4 (32-35 against 24 on the matrix cores), the
-# down matrix at batch 3-4 (35-39 against 25), q / k / v at batch 2 (17.6
-# against 12.9; 0.79 M codes).
+# (23.2 against 20.9) and 3-4 (32-35 against 25 in vq_rows_gemm), the
+# down matrix at batch 3-4 (35-39 against 28), q / k / v at batch 2 (17.6
+# against 12.9; 0.79 M codes), projections of one activation at batch 3-4
+# (three of 1024 x 2048 22.0-24.4 against 13.6 in vq_rows_gemm, gate + up
+# 40.1-42.0 against 39.1): there it only serves released planes and rows too
+# wide for vq_rows_gemm.
 SORTED_BATCH = True
 SORTED_BATCH_MIN_CODES = 8 << 20
 # PackedProjections at batch 2 on the sorted layout from this many codes on
@@ -89,6 +89,12 @@ def vq_matmul(xr, i0, i1, cb0, cb1, scale, out, n, out_dtype, y=None):
         b1 = min(B, b0 + SMALL_M_MAX)
         K.vq_gemm_small_m(xr[b0:b1], i0, i1, cb0, cb1, scale, out, n, 1.0, y=y[b0:b1])
     return y
+
+
+def _rows_ok(x2, n, rot):
+    """Whether x2 [B, n] takes vq_rows_gemm (rotation and product of all rows
+    in two launches): three rows or more of a width its packing holds."""
+    return x2.shape[0] >= 3 and n % 64 == 0 and n <= K.ROWS_GEMM_MAX_N and rot.hb >= 64
 
 
 class PackedLinear(nn.Module):
@@ -201,6 +207,9 @@ class PackedLinear(nn.Module):
             # one launch: every workgroup rotates x in LDS, then multiplies
             y = K.vq_gemv_rht(x2, [(i0, i1, self.scale, self.out)], cb0, cb1, self.n, self.rot._perm32,
                               self.rot._sign8, self.rot.hb, self.rot.scale, out_dtype=od)[0]
+        elif _rows_ok(x2, self.n, self.rot):
+            y = K.vq_rows_gemm(x2, [(i0, i1, self.scale, self.out)], cb0, cb1, self.n, self.rot._perm32,
+                               self.rot._sign8, self.rot.hb, self.rot.scale, act_dtype=self.act_dtype, out_dtype=od)[0]
         else:
             xr = self.rot.fwd(x2, out_dtype=self.act_dtype)
             y = vq_matmul(xr, i0, i1, cb0, cb1, self.scale, self.out, self.n, od)
@@ -220,11 +229,13 @@ class PackedProjections(nn.Module):
     projection's own forward gives (vq2/runtime.py:91-110, once per matrix
     there): with the sorted layout (the matrices hold
     ``SORTED_MIN_LAUNCH_CODES`` codes or more together) one sorted launch at
-    batch 1 and one sorted batch launch after the RHT at batch 3-4, and at
-    batch 2 with ``SORTED_BATCH2_LAUNCH_MIN_CODES`` codes or more (gate +
-    up); else one
-    gather-kernel launch with the RHT built in for batch <= 2; other batches
-    run each projection.  Up to 4 projections."""
+    batch 1 and one sorted batch launch after the RHT at batch 2 with
+    ``SORTED_BATCH2_LAUNCH_MIN_CODES`` codes or more (gate + up); else one
+    gather-kernel launch with the RHT built in for batch <= 2, and one
+    rotation and one product of all matrices from batch 3 on
+    (``kernels.vq_rows_gemm``; released planes or rows it does not take: the
+    sorted batch launch at batch 3-4, else each projection by itself).  Up to
+    4 projections."""
 
     def __init__(self, linears, sorted_layout=None):
         super().__init__()
@@ -267,12 +278,14 @@ class PackedProjections(nn.Module):
         i0, i1, cb0, cb1 = a._planes()
         od = out_dtype or x.dtype
         B = x2.shape[0]
+        rows = (_rows_ok(x2, a.n, a.rot) and not any(m.planes_released for m in lins)
+                and all(m.act_dtype == a.act_dtype for m in lins))
         if self.sorted is not None and B == 1 and cb0.dtype in (torch.float16, torch.bfloat16):
             xs, perm, sign, hb, sc = a._sorted_args(x2.reshape(-1))
             ys = K.vq_sorted_gemv(xs, [(sp, m.scale) for sp, m in zip(self.sorted, lins)], cb0, cb1, a.n, perm,
                                   sign, hb, sc, out_dtype=od)
         elif (SORTED_BATCH and self.sorted is not None and 2 <= B <= K.SORTED_BATCH_MAX
-              and (B >= 3 or self.codes >= SORTED_BATCH2_LAUNCH_MIN_CODES)
+              and (self.codes >= SORTED_BATCH2_LAUNCH_MIN_CODES if B == 2 else not rows)
               and cb0.dtype in (torch.float16, torch.bfloat16) and K.sorted_batch_fits(self.sorted, B)):
             xr = a.rot.fwd(x2, out_dtype=torch.float32)
             ys = K.vq_sorted_gemm_batch(xr, [(sp, m.scale) for sp, m in zip(self.sorted, lins)], cb0, cb1, a.n,
@@ -286,6 +299,9 @@ class PackedProjections(nn.Module):
                 mats.append((mi0, mi1, m.scale, m.out))
             ys = K.vq_gemv_rht(x2, mats, cb0, cb1, a.n, a.rot._perm32, a.rot._sign8, a.rot.hb, a.rot.scale,
                                out_dtype=od)
+        elif rows:
+            ys = K.vq_rows_gemm(x2, [(*m._planes()[:2], m.scale, m.out) for m in lins], cb0, cb1, a.n, a.rot._perm32,
+                                a.rot._sign8, a.rot.hb, a.rot.scale, act_dtype=a.act_dtype, out_dtype=od)
         else:
             return [m(x, out_dtype=out_dtype) for m in lins]
         return [y.view(*x.shape[:-1], m.out) for y, m in zip(ys, lins)]

@@ -160,6 +160,26 @@ int vq2_gemv_rht(const void* x, int x_dt, int64_t batch, int64_t x_stride,
                  int s2_kind, const void* cb0, const void* cb1, int cb_dt, int s_dt, int y_dt,
                  int64_t n, float rs, void* stream);
 
+/* Rotate and multiply for any number of activation rows, up to 4 matrices
+ * that share the activation, on the matrix cores:
+ *   xr[b] = RHT_fwd(x[b]) as in vq2_gemv_rht (hb == 0: x is rotated), rounded
+ *           to act_dt, then to fp16 under a power-of-two scale per row
+ *   segs[s].y[b, r] = (sum_k W_s[r, k] * xr[b, k]) * segs[s].scale[r] * rs
+ * Codebooks that are not fp16 are rounded to fp16; sums are fp32.  Two
+ * launches: the rotated rows go to the workspace in the order the product's
+ * matrix instructions read them.  Requires n % 64 == 0, n <= 8192, hb a power
+ * of two from 64 on (or 0), 16-byte aligned index planes; x needs no
+ * alignment.  The workspace (256-byte aligned, vq2_rows_gemm_workspace bytes;
+ * 0 for sizes the entry refuses; of segs it reads out_rows alone) may hold
+ * anything on entry.  Replaces Rot.fwd + F.linear of
+ * the PackedLinear fallback (vq2/runtime.py:82-89, 105-110). */
+size_t vq2_rows_gemm_workspace(int64_t batch, int64_t n, int n_seg, const vq2_seg* segs, int s2_kind, int cb_dt);
+int vq2_rows_gemm(const void* x, int x_dt, int64_t batch, int64_t x_stride,
+                  const int32_t* perm, const int8_t* sign, int64_t hb, float rht_scale, int act_dt,
+                  int n_seg, const vq2_seg* segs,
+                  int s2_kind, const void* cb0, const void* cb1, int cb_dt, int s_dt, int y_dt,
+                  int64_t n, float rs, void* workspace, size_t ws_bytes, void* stream);
+
 
 /* Grouped per-expert 2 bpw VQ GEMV over a device-resident expert pool:
  *   e = ids[k];  y[k, r] = (sum_g cb[pool[e, r, g]] . x_k[8g:8g+8]) * pool_scale[e, r] * rs
