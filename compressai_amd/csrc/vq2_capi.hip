@@ -352,6 +352,60 @@ int vq2_rows_gemm(const void* x, int x_dt, int64_t batch, int64_t x_stride, cons
     return rows_launch(c);
 }
 
+size_t vq2_moe_rows_workspace(int64_t tokens, int pairs, int64_t n_experts, int64_t hidden, int64_t inter, int cb_dt)
+{
+    MoeRowsCall c{};
+    c.tokens = tokens;
+    c.P = pairs;
+    c.n_experts = n_experts;
+    c.hidden = hidden;
+    c.inter = inter;
+    c.cb_dt = cb_dt;
+    return moe_rows_workspace_bytes(c);
+}
+
+int vq2_moe_rows(const void* h, int h_dt, int64_t tokens, int pairs, const void* ids, int ids_dt, const float* w,
+                 int64_t n_experts, int64_t hidden, int64_t inter, const int16_t* gate_up, const void* gate_up_scale,
+                 int gate_up_s_dt, const int16_t* down, const void* down_scale, int down_s_dt, const void* cb, int cb_dt,
+                 const vq2_rot_tables* rot_h, const vq2_rot_tables* rot_i, void* out, int out_dt, void* workspace,
+                 size_t ws_bytes, void* stream)
+{
+    clear_error();
+    CHECK(tokens >= 0, "vq2_moe_rows: negative token count");
+    if (tokens == 0) return VQ2_OK;
+    CHECK(h && ids && w && gate_up && gate_up_scale && down && down_scale && cb && rot_h && rot_i && out,
+          "vq2_moe_rows: NULL pointer argument");
+    CHECK(dt_ok(h_dt) && dt_ok(out_dt) && dt_ok(gate_up_s_dt) && dt_ok(down_s_dt), "vq2_moe_rows: bad dtype code");
+    CHECK(ids_dt == VQ2_ID_I32 || ids_dt == VQ2_ID_I64, "vq2_moe_rows: bad ids dtype");
+    MoeRowsCall c{};
+    c.h = h;
+    c.h_dt = h_dt;
+    c.tokens = tokens;
+    c.P = pairs;
+    c.ids = ids;
+    c.ids_i64 = ids_dt == VQ2_ID_I64;
+    c.w = w;
+    c.n_experts = n_experts;
+    c.hidden = hidden;
+    c.inter = inter;
+    c.gu_idx = gate_up;
+    c.gu_scale = gate_up_scale;
+    c.gu_s_dt = gate_up_s_dt;
+    c.dn_idx = down;
+    c.dn_scale = down_scale;
+    c.dn_s_dt = down_s_dt;
+    c.cb = cb;
+    c.cb_dt = cb_dt;
+    c.rot_h = SortedRot{rot_h->perm, rot_h->sign, rot_h->hb, rot_h->scale};
+    c.rot_i = SortedRot{rot_i->perm, rot_i->sign, rot_i->hb, rot_i->scale};
+    c.out = out;
+    c.out_dt = out_dt;
+    c.workspace = workspace;
+    c.ws_bytes = ws_bytes;
+    c.stream = stream;
+    return moe_rows_launch(c);
+}
+
 int vq2_moe_grouped(const void* x, int x_dt, int64_t x_pair_stride, int64_t pairs_per_x, const void* ids,
                     int ids_dt, int64_t n_pairs, const int16_t* pool, int64_t n_experts, const void* cb, int cb_dt,
                     const void* pool_scale, int s_dt, void* y, int y_dt, int64_t y_pair_stride, int64_t out_rows,

@@ -291,6 +291,39 @@ struct SortedMoeCall {
     void* stream;
 };
 
+// MoE experts for many tokens over the reference-layout pools
+// (vq2_moe_rows.hip).
+struct MoeRowsCall {
+    const void* h;
+    int h_dt;
+    int64_t tokens;
+    int P;  // pairs per token
+    const void* ids;
+    int ids_i64;
+    const float* w;
+    int64_t n_experts;
+    int64_t hidden;
+    int64_t inter;
+    const int16_t* gu_idx;
+    const void* gu_scale;
+    int gu_s_dt;
+    const int16_t* dn_idx;
+    const void* dn_scale;
+    int dn_s_dt;
+    const void* cb;
+    int cb_dt;
+    SortedRot rot_h;
+    SortedRot rot_i;
+    void* out;
+    int out_dt;
+    void* workspace;
+    size_t ws_bytes;
+    void* stream;
+};
+
+size_t moe_rows_workspace_bytes(const MoeRowsCall& c);  // 0 for sizes that moe_rows_launch refuses
+int moe_rows_launch(const MoeRowsCall& c);
+
 size_t sorted_moe_workspace_bytes(int64_t n_pairs, int64_t hidden, int64_t inter, int slices_gu, int slices_dn);
 int sorted_moe_launch(const SortedMoeCall& c);
 

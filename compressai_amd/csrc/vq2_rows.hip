@@ -48,13 +48,12 @@
 
 #include "vq2_common.hpp"
 #include "vq2_internal.hpp"
+#include "vq2_rot_row.hpp"
 
 namespace vq2 {
 
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
 constexpr int RW_TILE_G = 32;      // groups per k tile
-constexpr int RW_PACK_MAX = 1024;  // threads of a packing workgroup: one per group of its row
+constexpr int RW_PACK_MAX = ROT_ROW_MAX_T;
 constexpr int64_t RW_MAX_N = 8 * RW_PACK_MAX;
 constexpr int RW_CB_ROWS = 65536;
 
@@ -122,12 +121,7 @@ __device__ __forceinline__ void rows_cvt_codebook(const RowsPackArgs& a, int64_t
     dst[i] = h;
 }
 
-// Workgroup b < m: row b.  Thread t holds the 8 values of group t: value bits
-// 0-2 are in its registers, bits 3-8 across the lanes of its wave, 9-10 and
-// 11-12 across waves (one radix-4 exchange through LDS each).  The stages run
-// from bit 0 up, as in rht_kernel.  One group a thread keeps a 6144-value row
-// as fast as a 2048-value one: with 256 threads and three groups each it took
-// twice as long (11.4 against 5.8 us), serial latency on one wave per SIMD.
+// Workgroup b < m: row b, one thread per group (vq2_rot_row.hpp).
 __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackArgs a)
 {
     extern __shared__ __align__(16) float s_x[];  // the row; later the exchanges
@@ -149,104 +143,17 @@ __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackAr
     // this thread's permutation and sign words, then the row into LDS
     int32_t pw[8];
     uint32_t sg[2];
-    if (rot) {
-        const int gc = g_ok ? tid : 0;
-        if (a.perm) {
-            const u32x4 p0 = *((const u32x4*)a.perm + 2 * gc), p1 = *((const u32x4*)a.perm + 2 * gc + 1);
-#pragma unroll
-            for (int k = 0; k < 4; k++) { pw[k] = (int32_t)p0[k]; pw[4 + k] = (int32_t)p1[k]; }
-        } else {
-#pragma unroll
-            for (int k = 0; k < 8; k++) pw[k] = gc * 8 + k;
-        }
-        if (a.sign) {
-            const u32x2 w = *((const u32x2*)a.sign + gc);
-            sg[0] = w.x;
-            sg[1] = w.y;
-        } else {
-            sg[0] = sg[1] = 0x01010101u;
-        }
-    }
-    const int64_t x0 = row * a.x_stride;
-    if (a.x_vec) {
-        if (a.x_dt == VQ2_DT_F32) {
-            const u32x4* xr = (const u32x4*)((const float*)a.x + x0);
-            for (int c = tid; c < a.n / 4; c += T) *((u32x4*)s_x + c) = xr[c];
-        } else if (g_ok) {
-            const u32x4 w = *((const u32x4*)((const uint16_t*)a.x + x0) + tid);
-#pragma unroll
-            for (int k = 0; k < 4; k++) {
-                s_x[tid * 8 + 2 * k] = a.x_dt == VQ2_DT_BF16 ? __uint_as_float(w[k] << 16)
-                                                             : f16_bits_to_f32((uint16_t)(w[k] & 0xFFFFu));
-                s_x[tid * 8 + 2 * k + 1] = a.x_dt == VQ2_DT_BF16 ? __uint_as_float(w[k] & 0xFFFF0000u)
-                                                                 : f16_bits_to_f32((uint16_t)(w[k] >> 16));
-            }
-        }
-    } else {
-        for (int i = tid; i < a.n; i += T) s_x[i] = load_as_f32(a.x, a.x_dt, x0 + i);
-    }
+    if (rot) rot_tables(a.perm, a.sign, g_ok ? tid : 0, pw, sg);
+    rot_stage_row(a.x, a.x_dt, a.x_vec, row * a.x_stride, a.n, s_x, tid, T);
     __syncthreads();
 
     float v[8];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        if (!g_ok) {
-            v[k] = 0.0f;
-        } else if (!rot) {
-            v[k] = s_x[tid * 8 + k];
-        } else {
-            const bool bad = (uint32_t)pw[k] >= (uint32_t)a.n;  // not a permutation: poison, in bounds
-            const float s = (float)(int8_t)(sg[k >> 2] >> (8 * (k & 3)));
-            v[k] = bad ? __builtin_nanf("") : s_x[bad ? 0 : pw[k]] * s;
-        }
-    }
     if (rot) {
+        rot_gather(s_x, pw, sg, a.n, g_ok, v);
+        rot_transform(v, s_x, tid, T, a.hb_log2);
+    } else {
 #pragma unroll
-        for (int h = 1; h < 8; h <<= 1)
-#pragma unroll
-            for (int k = 0; k < 8; k++)
-                if ((k & h) == 0) {
-                    const float p = v[k], q = v[k | h];
-                    v[k] = p + q;
-                    v[k | h] = p - q;
-                }
-        auto stage = [&](int bit, auto partner) {
-            if (a.hb_log2 > bit) {
-                const bool up = (lane >> (bit - 3)) & 1;
-#pragma unroll
-                for (int k = 0; k < 8; k++) {
-                    const float o = partner(v[k]);
-                    v[k] = up ? o - v[k] : v[k] + o;
-                }
-            }
-        };
-        stage(3, [](float f) { return dpp_xor1(f); });
-        stage(4, [](float f) { return dpp_xor2(f); });
-        stage(5, [](float f) { return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(f), 0x101F)); });
-        stage(6, [](float f) { return __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(f), 0x201F)); });
-        stage(7, [](float f) { return swz_xor16(f); });
-        stage(8, [](float f) { return xor32(f); });
-        // bits b and b + 1 across waves: component k of group t at k * T + t
-        for (int b = 9; b < a.hb_log2; b += 2) {
-            const int d = 1 << (b - 3);
-            __syncthreads();
-#pragma unroll
-            for (int k = 0; k < 8; k++) s_x[k * T + tid] = v[k];
-            __syncthreads();
-            const bool u0 = tid & d, u1 = tid & (2 * d), two = a.hb_log2 > b + 1;
-#pragma unroll
-            for (int k = 0; k < 8; k++) {
-                const float o = s_x[k * T + (tid ^ d)];
-                const float r = u0 ? o - v[k] : v[k] + o;
-                if (two) {
-                    const float p2 = s_x[k * T + (tid ^ (2 * d))], o2 = s_x[k * T + (tid ^ (3 * d))];
-                    const float r2 = u0 ? o2 - p2 : p2 + o2;
-                    v[k] = u1 ? r2 - r : r + r2;
-                } else {
-                    v[k] = r;
-                }
-            }
-        }
+        for (int k = 0; k < 8; k++) v[k] = g_ok ? s_x[tid * 8 + k] : 0.0f;
     }
     float am = 0.0f;
 #pragma unroll
@@ -254,14 +161,7 @@ __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackAr
         if (rot) v[k] = rows_round_act(v[k] * a.scale, a.act_dt);
         am = fmaxf(am, fabsf(v[k]));  // skips NaN, which reaches its output row through the product
     }
-    am = wave_max_all(am);
-    if (lane == 0) s_max[wave] = am;
-    __syncthreads();
-    for (int w = 0; w < T / 64; w++) am = fmaxf(am, s_max[w]);
-    // the row's largest value into [2^14, 2^15): exact, far below 65504; a
-    // row of zeros or with an infinity keeps scale 1
-    const uint32_t ab = __float_as_uint(am);
-    const int e = ab != 0u && ab < 0x7F800000u ? 14 - ilogbf(am) : 0;
+    const int e = rot_row_exponent(am, s_max, tid, T);
     if (tid == 0) a.e[row] = e;
     const int kt = tid / RW_TILE_G, t = tid & 7, q = (tid >> 3) & 3;
     if (kt >= a.kt) return;

@@ -1038,6 +1038,64 @@ def vq_sorted_moe(h, gate_up: SortedPool, gu_scale, down: SortedPool, dn_scale, 
     return out
 
 
+# Largest pool vq_moe_rows sorts pairs for, and its token limit.
+MOE_ROWS_MAX_EXPERTS = 4096
+MOE_ROWS_MAX_TOKENS = 65535
+MOE_ROWS_MIN_PAIRS = 256
+
+
+def moe_rows_faster(pairs, n_experts, hidden, inter) -> bool:
+    """Whether vq_moe_rows takes less time than the one-pair kernels: those
+    gather ~480 codes a ns for each pair, it ~200 a ns for each expert of the
+    pool (all touched at worst) behind ~30 us of launches.  Measured on MI355X
+    at the 35B shape (257 pool entries, 9 pairs a token, us a layer, one-pair
+    against grouped): 56 tokens 414 / 458, 64 471 / 471, 72 521 / 493, 128
+    896 / 509, 512 3526 / 609; the line lies at 73 tokens there.  Small pools
+    switch from MOE_ROWS_MIN_PAIRS pairs on (17 entries, 5 pairs a token, 52
+    tokens 246 / 82); fewer pairs stay on the one-pair kernels, as decode
+    batches do at the 35B shape."""
+    codes = 3 * hidden * inter // 8
+    return pairs >= MOE_ROWS_MIN_PAIRS and pairs * codes / 480e3 > n_experts * codes / 200e3 + 30.0
+
+
+def vq_moe_rows(h, ids, w, gate_up_idx, gate_up_scale, down_idx, down_scale, cb, rot_h, rot_i, *, out=None,
+                out_dtype=torch.float32):
+    """The experts of an MoE layer for many tokens, over the reference-layout
+    pools gate_up_idx [E, 2I, H/8] and down_idx [E, H, I/8]: the pairs of one
+    expert share its gathered centroids on the matrix cores (five launches).
+    h [T, H], ids [T, P] int32 / int64, w fp32 [T, P]; rot_h / rot_i: (perm
+    int32, sign int8, hb, scale).  Returns out [T, H]."""
+    if gate_up_idx.dim() != 3 or down_idx.dim() != 3:
+        raise Vq2Error("vq_moe_rows: pools must be [E, rows, ng]")
+    E, H, I = gate_up_idx.shape[0], gate_up_idx.shape[2] * 8, down_idx.shape[2] * 8
+    gu = _moe_checks(gate_up_idx, gate_up_scale, 2 * I, H // 8, "gate_up_idx")
+    dn = _moe_checks(down_idx, down_scale, H, I // 8, "down_idx")
+    if dn.shape[0] != E:
+        raise Vq2Error("vq_moe_rows: gate_up and down pools of different sizes")
+    rh, ri = _rot_tables(rot_h, H, "rot_h"), _rot_tables(rot_i, I, "rot_i")
+    dev = _dev(h, ids, w, gu, gate_up_scale, dn, down_scale, cb, rot_h[0], rot_h[1], rot_i[0], rot_i[1], out)
+    _contig(cb, "cb")
+    if cb.dim() != 2 or cb.shape[0] < 65536 or cb.shape[1] != 8 or cb.dtype not in (torch.float16, torch.bfloat16):
+        raise Vq2Error("vq_moe_rows: cb must be an fp16 / bf16 [65536, 8] codebook")
+    h2 = _contig(h, "h").reshape(-1, H)
+    T = h2.shape[0]
+    ids2, ids_dt = _ids(ids.reshape(T, -1))
+    P = ids2.shape[1]
+    w2 = _contig(w, "w")
+    if w2.dtype != torch.float32 or w2.numel() != T * P:
+        raise Vq2Error("vq_moe_rows: w must be fp32 [T, P]")
+    if out is None:
+        out = torch.empty((T, H), dtype=out_dtype, device=dev)
+    elif out.numel() != T * H or not out.is_contiguous():
+        raise Vq2Error(f"out must be a contiguous [{T}, {H}]")
+    cdt = _dt(cb, "cb")
+    ws = torch.empty(_lib.load().vq2_moe_rows_workspace(T, P, E, H, I, cdt), dtype=torch.uint8, device=dev)
+    _lib.call("vq2_moe_rows", _p(h2), _dt(h2, "h"), T, P, _p(ids2), ids_dt, _p(w2), E, H, I, _p(gu), _p(gate_up_scale),
+              _dt(gate_up_scale, "scale"), _p(dn), _p(down_scale), _dt(down_scale, "scale"), _p(cb), cdt,
+              ctypes.byref(rh), ctypes.byref(ri), _p(out), _dt(out, "out"), _p(ws), ws.numel(), _stream(dev))
+    return out
+
+
 # -------------------------------------------------------------- grouped MoE
 def _moe_checks(pool, scale, OUT, NG, what):
     pool = _idx16(pool, what)

@@ -33,8 +33,11 @@ run the experts over it, so a wave's centroid gathers share codebook lines:
 at hidden 2048 / intermediate 512 (the 35B-A3B shape) gate_up (router built
 in for ``MoELayer``) and down (SwiGLU + RHT in its prologue) are one launch,
 followed by the combine launch; other widths take a separate down launch.
-The reference pools stay the public format and serve ``act_dtype`` bf16,
-more than 256 routed experts and the paged feed; a caller that needs none
+With many tokens (``kernels.moe_rows_faster``, from 73 on at the 35B shape) the
+pairs of one expert are grouped and share its gathered centroids on the matrix
+cores (``kernels.vq_moe_rows``), over the reference pools.
+The reference pools stay the public format and serve many tokens,
+``act_dtype`` bf16, more than 256 routed experts and the paged feed; a caller that needs none
 of these frees them with ``release_reference_pools()`` (resident index
 memory then ~3.06 instead of ~5.06 bytes per code; ``sorted_layout=False``
 keeps only the 2-byte pools, on the gather kernels).  The down pool is
@@ -171,6 +174,22 @@ class ResidentMoEExperts(nn.Module):
         rh, ri = self.rot_h, self.rot_i
         return (rh._perm32, rh._sign8, rh.hb, rh.scale), (ri._perm32, ri._sign8, ri.hb, ri.scale)
 
+    def _rows_ok(self, h, pairs):
+        """Whether h [T, H] with that many pairs takes kernels.vq_moe_rows:
+        enough pairs to share the experts' codes, the reference pools there
+        in the form it reads, and what the sorted path takes besides."""
+        gu, dn = self.gate_up_idx, self.down_idx
+        return (gu is not None and h.shape[0] <= K.MOE_ROWS_MAX_TOKENS
+                and self.num_experts <= K.MOE_ROWS_MAX_EXPERTS and max(self.hidden_dim, self.intermediate_dim) <= 8192
+                and min(self.rot_h.hb, self.rot_i.hb) >= 64 and gu.is_contiguous() and dn.is_contiguous()
+                and all(t.data_ptr() % 16 == 0 for t in (gu, dn, h))
+                and K.moe_rows_faster(pairs, self.num_experts, self.hidden_dim, self.intermediate_dim))
+
+    def _rows(self, h, ids, w, out=None):
+        rh, ri = self._rots()
+        return K.vq_moe_rows(h, ids, w, self.gate_up_idx, self.gate_up_scale, self.down_idx, self.down_scale, self.cb16,
+                             rh, ri, out=out, out_dtype=self.out_dtype or torch.float32)
+
     def nbytes(self):
         """Resident bytes: index pools, scales and the sorted copies."""
         own = sum(t.numel() * t.element_size() for t in (self.gate_up_idx, self.gate_up_scale, self.down_idx,
@@ -180,9 +199,12 @@ class ResidentMoEExperts(nn.Module):
     def experts(self, h, ids, w, out=None):
         """h [T, H] (unrotated hidden states), ids [T, P] int32/int64,
         w fp32 [T, P] -> [T, H].  Sorted pools: gate_up and down (SwiGLU +
-        RHT in its prologue) in one launch at the 35B shape, then the combine;
+        RHT in its prologue) in one launch at the 35B shape, then the combine,
+        or with many pairs the reference pools grouped by expert (_rows_ok);
         otherwise two launches, gate_up with the H-point RHT fused, then
         SwiGLU + I-point RHT + down + weighted combine."""
+        if self.sorted_gu is not None and self._rows_ok(h, ids.numel()):
+            return self._rows(h, ids, w, out)
         if self.sorted_gu is not None:
             rh, ri = self._rots()
             return K.vq_sorted_moe(h, self.sorted_gu, self.gate_up_scale, self._down_pool(h.shape[0]), self.down_scale,
@@ -237,13 +259,18 @@ class MoELayer(nn.Module):
 
     def forward(self, h, router_logits):
         """Sorted pools: router + gate_up and down (SwiGLU + RHT prologue) in
-        one launch at the 35B shape, then the combine.  Otherwise two
+        one launch at the 35B shape, then the combine; with many tokens the
+        router, then the experts grouped (_rows_ok).  Otherwise two
         launches: router + gate_up (+ RHT), then SwiGLU + RHT + down +
         combine."""
         m = self.experts_mod
         h2 = h.reshape(-1, m.hidden_dim).contiguous()
         T = h2.shape[0]
         if m.sorted_gu is not None and self.n_routed <= 256:
+            # (calls that the sorted path refuses are left to it)
+            if (self.n_routed < m.num_experts and router_logits.numel() <= 256 * T and self.top_k <= 64
+                    and m._rows_ok(h2, T * (self.top_k + 1))):
+                return m._rows(h2, *self.route(h2, router_logits.reshape(T, -1)))
             rh, ri = m._rots()
             out, _, _ = K.vq_sorted_moe(h2, m.sorted_gu, m.gate_up_scale, m._down_pool(T), m.down_scale, m.cb16, rh, ri,
                                         logits=router_logits.reshape(T, -1), top_k=self.top_k,

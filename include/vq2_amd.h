@@ -578,6 +578,28 @@ int vq2_sorted_moe(const void* h, int h_dt, int64_t tokens, int pairs_per_token,
                    const vq2_rot_tables* rot_h, const vq2_rot_tables* rot_i, void* out, int out_dt,
                    int slices_gu, int slices_dn, void* workspace, size_t ws_bytes, void* stream);
 
+/* The experts of an MoE layer for many tokens, over the reference-layout
+ * pools: out[t] = sum_k w[t, k] * VQ(down[e]) RHT_I(silu(gu[:I]) * gu[I:]),
+ * gu = VQ(gate_up[e]) RHT_H(h[t]), e = ids[t, k].  The pairs are grouped by
+ * expert on the device and an expert's codes are gathered once per 32 or 64
+ * of its pairs, for the matrix cores: the fp32 activation is split into three
+ * 8-bit addends (bf16 for bf16 codebooks; fp16 under a power-of-two scale per
+ * row for fp16 ones); sums are fp32.  An id outside [0, n_experts) gives
+ * NaN.  hidden and inter: multiples of 64 up to 8192, their rotation blocks
+ * powers of two from 64 on; n_experts at most 4096, tokens at most 65535;
+ * pools and codebook 16-byte aligned.  gate_up [n_experts, 2 inter, hidden/8],
+ * down [n_experts, hidden, inter/8], scales [n_experts, rows].  Five launches;
+ * the workspace (256-byte aligned, vq2_moe_rows_workspace bytes; 0 for sizes
+ * the entry refuses) may hold anything on entry.  Replaces
+ * PagedMoEExpert.forward (vq2/paged_runtime.py:439-568). */
+size_t vq2_moe_rows_workspace(int64_t tokens, int pairs, int64_t n_experts, int64_t hidden, int64_t inter, int cb_dt);
+int vq2_moe_rows(const void* h, int h_dt, int64_t tokens, int pairs, const void* ids, int ids_dt, const float* w,
+                 int64_t n_experts, int64_t hidden, int64_t inter,
+                 const int16_t* gate_up, const void* gate_up_scale, int gate_up_s_dt,
+                 const int16_t* down, const void* down_scale, int down_s_dt, const void* cb, int cb_dt,
+                 const vq2_rot_tables* rot_h, const vq2_rot_tables* rot_i,
+                 void* out, int out_dt, void* workspace, size_t ws_bytes, void* stream);
+
 /* ---- Device-resident expert pager ---------------------------------------
  * The slot tables of a paged expert pool on the device: slot_of
  * [n_experts] (slot or -1), expert_of [capacity] (expert or -1), stamp
