@@ -4,13 +4,14 @@
 //   y_s[m, r] = (sum_k RHT(x)[m, k] * W_s[r, k]) * scale_s[r] * rs,
 //   W[r, 8g + j] = cb0[i0[r, g]][j] (+ cb1[i1[r, g]][j]).
 //
-// Two launches for any number of rows:
+// Two or three launches for any number of rows:
 //  1. rows_pack_kernel: one workgroup per activation row rotates it (or takes
 //     it rotated), finds the row's power-of-two scale and writes it as fp16
 //     in the order the second launch's matrix instructions read (below).
 //     Codebooks that are not fp16 are rounded to fp16 by further workgroups
 //     of the same launch, so the second launch gathers 16 bytes a code.
-//  2. rows_gemm_kernel: the product.
+//  2. rows_gemm_kernel, or for many rows rows_wide_kernel (and rows_sum_kernel
+//     where its k tiles are shared): the product.
 //
 // Why two launches and this layout.  The products are bound by the random
 // 16-byte centroid gathers, which the L2s serve at ~240 G/s whatever else the
@@ -26,7 +27,7 @@
 // reduce launch): 2048 x 6144 at 4 bpw, 16 rows 29.3 -> 27.5; 6144 x 2048 at
 // 4 bpw, 64 rows 37.1 -> 31.2; two 6144 x 2048 at 3 bpw, 64 rows, bf16
 // 64.2 -> 38.6; 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5, 1024 rows
-// 264.8 -> 73.8.  Bound by the gathers (13 us of the 4 bpw calls) and, below
+// 264.8 -> 50.4; two 6144 x 2048 at 4 bpw, 1024 rows 981 -> 192.  Bound by the gathers (13 us of the 4 bpw calls) and, below
 // about a million codes, by the two launches' latency (~12 us).
 //
 // Fragment layout: v_mfma_f32_16x16x32_f16 takes 8 consecutive k of row
@@ -198,6 +199,7 @@ struct RowsArgs {
     int nz;  // workgroups that share them (gridDim.z); nc is 1 then
     float* part;    // nz > 1: [row block][column tile][nz][16 MT][16 NT] sums
     uint32_t* cnt;  // nz > 1: arrivals per [row block][column tile], zero
+    int tiles;      // column tiles of all matrices
     RowsSeg seg[4];
 };
 
@@ -233,6 +235,8 @@ __device__ __forceinline__ const RowsSeg& rows_seg(const RowsArgs& a, int tile)
 }
 
 constexpr int RW_MAX_WAVES = 16;
+constexpr int RW_MAX_MT = 4;     // 16-row tiles of a wave of rows_gemm_kernel
+constexpr int RW_WIDE_WAVES = 4; // waves of a rows_wide_kernel workgroup
 constexpr int RW_MAX_Z = 4;  // workgroups that share a tile's k tiles
 
 // Up to 16 * MT rows: a workgroup is nc column tiles of 16 * NT columns x kw
@@ -372,11 +376,185 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     }
 }
 
+// Many rows: a workgroup is 4 waves of 16 columns x 16 * MT rows and walks
+// all k tiles of its share (blockIdx.z of nz).  Per stage of TS steps the waves
+// gather their own operands into registers, a stage ahead, and stage the rows'
+// packed operands in LDS for all of them, two buffers in turn.  So a code is
+// gathered once per 128 or 256 rows instead of 64.  Bound by those gathers and,
+// as a wave reads every operand of the rows from LDS for its 16 columns, by
+// the LDS rate (with all codes alike, two 6144 x 2048 matrices at 4 bpw and
+// 1024 rows take 133 of 192 us).  Measured there, us a call: 8 waves and 4
+// steps a stage 208, 8 and 2 205, 4 and 2 192; 32 columns a wave, which halves
+// the LDS reads, spills at 256 rows (266), and so do 512 rows (216).
+template <int S2, int MT, int TS>
+__global__ void __launch_bounds__(64 * RW_WIDE_WAVES, 2) rows_wide_kernel(const RowsArgs a)
+{
+    touch_kernargs(a);
+    constexpr int NW = RW_WIDE_WAVES;
+    constexpr int HS = 8 / TS, NF = MT * TS;  // stages of a k tile, operands of a stage
+    constexpr int NL = (NF + NW - 1) / NW;    // operands a wave stages
+    static_assert(HS % 2 == 0, "two buffers in turn");
+    extern __shared__ __align__(16) half8_t s_wide[];
+    __shared__ half8_t s_c1[S2 == VQ2_S2_U8 ? 256 : 1];
+    half8_t (*s_a)[NF][64] = (half8_t (*)[NF][64])s_wide;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nl = lane & 15, q = lane >> 4;
+    const int tile = (int)blockIdx.x * NW + wave;
+    const RowsSeg& sg = rows_seg(a, tile);
+    const int col = (tile - sg.tile0) * 16 + nl;  // may lie past the last matrix's rows
+    const bool col_ok = col < sg.rows;
+    const int mt0 = (int)blockIdx.y * MT, mt_last = (a.m - 1) >> 4;
+    const int kt0 = (int)((int64_t)a.kt * blockIdx.z / a.nz), kt1 = (int)((int64_t)a.kt * (blockIdx.z + 1) / a.nz);
+    const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int64_t rowoff = (int64_t)(col_ok ? col : 0) * a.ng;
+
+    RowCodes<S2> c0, c1;
+    auto load_codes = [&](RowCodes<S2>& c, int kt) {
+        const int g = min(kt, a.kt - 1) * RW_TILE_G + q * 8;
+        c.load(sg, rowoff + (g < a.ng ? g : 0));
+    };
+    load_codes(c0, kt0);
+    if constexpr (S2 == VQ2_S2_U8) {
+        for (int i = tid; i < 256; i += 64 * NW) s_c1[i] = a.cb1[i];
+        __syncthreads();
+    }
+
+    // this wave stages the operands f = wave + NW i of every stage: row tile
+    // f / TS, step f % TS
+    const half8_t* src[NL];
+#pragma unroll
+    for (int i = 0; i < NL; i++) {
+        const int f = min(wave + NW * i, NF - 1);
+        src[i] = a.a + (int64_t)min(mt0 + f / TS, mt_last) * a.kt * 512 + f % TS * 64;
+    }
+    half8_t sa[NL];
+    auto load_a = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < NL; i++) sa[i] = (src[i] + stage * (64 * TS))[(uint32_t)lane];
+    };
+    f32x4_t acc[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    half8_t b0[TS], b1[TS], n0[TS], n1[TS];
+    auto gather = [&](const RowCodes<S2>& c, int t0, half8_t (&g0)[TS], half8_t (&g1)[TS]) {
+#pragma unroll
+        for (int j = 0; j < TS; j++) {
+            g0[j] = a.cb0[c.c0(t0 + j)];
+            if constexpr (S2 == VQ2_S2_U16) g1[j] = a.cb1[c.c1(t0 + j)];
+            if constexpr (S2 == VQ2_S2_U8) g1[j] = s_c1[c.c1(t0 + j)];
+        }
+    };
+    load_a(kt0 * HS);
+    gather(c0, 0, b0, b1);
+    load_codes(c1, kt0 + 1);
+
+    for (int kt = kt0; kt < kt1; kt++) {
+        const bool g_ok = kt * RW_TILE_G + q * 8 < a.ng;
+#pragma unroll
+        for (int h = 0; h < HS; h++) {
+#pragma unroll
+            for (int i = 0; i < NL; i++)
+                if (NF % NW == 0 || wave + NW * i < NF) s_a[h & 1][wave + NW * i][lane] = sa[i];
+            __syncthreads();
+            if (h + 1 < HS || kt + 1 < kt1) {
+                load_a(kt * HS + h + 1);
+                if (h + 1 < HS) gather(c0, (h + 1) * TS, n0, n1);
+                else gather(c1, 0, n0, n1);
+            }
+            if (h + 1 == HS) {
+                c0 = c1;
+                load_codes(c1, kt + 2);
+            }
+            // operands in batches, the next one's LDS reads before this one's
+            // products (left to itself the compiler waits for each read and
+            // issues the stage's loads after its products)
+            __builtin_amdgcn_sched_barrier(0);
+            constexpr int FB = 4, NB = NF / FB;
+            half8_t fr[2][FB];
+            // operand u: step u / MT, row tile u % MT
+            auto read = [&](int bt, half8_t (&r)[FB]) {
+#pragma unroll
+                for (int f = 0; f < FB; f++) {
+                    const int u = bt * FB + f;
+                    r[f] = s_a[h & 1][u % MT * TS + u / MT][lane];
+                }
+            };
+            read(0, fr[0]);
+#pragma unroll
+            for (int j = 0; j < TS; j++) {
+                b0[j] = g_ok ? b0[j] : zero8;
+                if constexpr (S2 != VQ2_S2_NONE) b1[j] = g_ok ? b1[j] : zero8;
+            }
+#pragma unroll
+            for (int bt = 0; bt < NB; bt++) {
+                if (bt + 1 < NB) read(bt + 1, fr[(bt + 1) & 1]);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int f = 0; f < FB; f++) {
+                    const int i = (bt * FB + f) % MT, j = (bt * FB + f) / MT;
+                    acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[bt & 1][f], b0[j], acc[i], 0, 0, 0);
+                }
+                if constexpr (S2 != VQ2_S2_NONE) {
+#pragma unroll
+                    for (int f = 0; f < FB; f++) {
+                        const int i = (bt * FB + f) % MT, j = (bt * FB + f) / MT;
+                        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[bt & 1][f], b1[j], acc[i], 0, 0, 0);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int j = 0; j < TS; j++) {
+                b0[j] = n0[j];
+                b1[j] = n1[j];
+            }
+        }
+    }
+
+    if (!col_ok) return;
+    const float s = a.nz > 1 ? 0.0f : load_as_f32(sg.scale, a.s_dt, col);
+#pragma unroll
+    for (int u = 0; u < MT * 4; u++) {
+        const int i = u / 4, e = u % 4;
+        const int row = (mt0 + i) * 16 + q * 4 + e;
+        if (row >= a.m) continue;
+        const float p = ldexpf(acc[i][e], -a.e[row]);
+        if (a.nz > 1)
+            a.part[((int64_t)blockIdx.z * a.m + row) * (a.tiles * 16) + tile * 16 + nl] = p;
+        else
+            store_from_f32(sg.y, a.y_dt, (int64_t)row * sg.y_stride + col, (p * s) * a.rs);
+    }
+}
+
+// y = (the shares of the k tiles added in order) * scale * rs, for nz > 1
+__global__ void __launch_bounds__(256) rows_sum_kernel(const RowsArgs a)
+{
+    const int c4 = (int)blockIdx.x * 256 + threadIdx.x, row = blockIdx.y;
+    if (c4 >= a.tiles * 4) return;
+    const int64_t ld = (int64_t)a.tiles * 16;
+    const float* p = a.part + row * ld + c4 * 4;
+    f32x4_t v[RW_MAX_Z], sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int z = 0; z < RW_MAX_Z; z++) v[z] = *(const f32x4_t*)(p + (int64_t)min(z, a.nz - 1) * a.m * ld);
+#pragma unroll
+    for (int z = 0; z < RW_MAX_Z; z++)
+        if (z < a.nz) sum += v[z];
+    const int tile = c4 / 4;
+    const RowsSeg& sg = rows_seg(a, tile);
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const int col = (tile - sg.tile0) * 16 + (c4 % 4) * 4 + k;
+        if (col < sg.rows)
+            store_from_f32(sg.y, a.y_dt, (int64_t)row * sg.y_stride + col, (sum[k] * load_as_f32(sg.scale, a.s_dt, col)) * a.rs);
+    }
+}
+
 // ------------------------------------------------------------------ launch
 struct RowsPlan {
     int kt;
     int mt, nt;        // 16-row and 16-column tiles of a wave
     int kw, nc, nz;    // waves and workgroups over a column tile's k tiles; column tiles of a workgroup
+    int wide;          // rows_wide_kernel
     int64_t tiles;     // column tiles of all matrices
     int64_t grid_x, grid_y;
     // workspace: arrival counters, the rows' exponents, the packed
@@ -386,11 +564,53 @@ struct RowsPlan {
 
 static size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 
+// Above 64 rows: rows_wide_kernel where a model of both kernels puts it ahead.
+// L2 requests are what both wait for: a gather per code and row block, and the
+// packed activation's lines, read once per 16 columns (rows_gemm_kernel) or
+// per workgroup of 64 (rows_wide_kernel).  Rates in requests a ns, measured
+// (MI355X): rows_gemm_kernel 235; rows_wide_kernel a workgroup 1.0 with 128
+// rows and 0.75 with 256, all of them 200 and 160; nz > 1 adds the partials'
+// launch (4 us) and their traffic (5 TB/s).  Over nine shapes and 65 to 1024
+// rows the choice is within 10 % of the fastest of the seven (us a call, rows
+// x n, bits, activation rows: rows_gemm / chosen): 2 x 6144 x 2048, 4, 100
+// rows 77 / 53, 1024 rows 545 / 196; 2048 x 6144, 4, 256 rows 83 / 61, 1024
+// 299 / 124; three of 1024 x 2048, 2, 333 rows 45 / 39, 1024 103 / 59; 512 x
+// 2048, 2, stays (1024 rows 31.5, the best wide plan 35).
+static void rows_plan_wide(const RowsCall& c, RowsPlan& p)
+{
+    const double stages = c.s2 == VQ2_S2_U16 ? 2 : 1, m = (double)c.m;
+    double codes = 0, rows = 0;
+    for (int s = 0; s < c.nseg; s++) rows += (double)c.seg[s].rows;
+    codes = rows * (double)(c.n / 8) * stages;
+    const double a_lines = m * (double)c.n * 2 / 128;
+    const double t_rows = (codes * (double)p.grid_y + a_lines * (double)p.tiles) / 235e3;
+    double best = t_rows;
+    const int64_t blocks = (p.tiles + RW_WIDE_WAVES - 1) / RW_WIDE_WAVES;
+    for (int mt = 8; mt <= 16; mt += 8) {
+        const int64_t rb = (c.m + 16 * mt - 1) / (16 * mt);
+        const double req = codes * (double)rb + a_lines * (double)blocks;
+        for (int nz = 1; nz <= std::min(RW_MAX_Z, p.kt); nz *= 2) {
+            const double rate = std::min((double)(blocks * rb * nz) * (mt == 8 ? 1.0 : 0.75), mt == 8 ? 200.0 : 160.0);
+            const double t = req / (rate * 1e3) + (nz > 1 ? 4.0 + nz * m * rows * 8 / 5e6 : 0.0) + 1.0;
+            if (t >= best) continue;
+            best = t;
+            p.wide = 1;
+            p.mt = mt;
+            p.nz = nz;
+            p.nc = RW_WIDE_WAVES;
+            p.kw = 1;
+            p.grid_y = rb;
+        }
+    }
+}
+
 static RowsPlan rows_plan(const RowsCall& c)
 {
     RowsPlan p{};
     p.kt = (int)((c.n / 8 + RW_TILE_G - 1) / RW_TILE_G);
-    p.mt = (int)std::min<int64_t>(4, (c.m + 15) / 16);
+    // row blocks of at most 64 rows, as even as whole tiles allow
+    const int64_t mtiles = (c.m + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
+    p.mt = (int)((mtiles + blocks - 1) / blocks);
     p.nt = 1;
     for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 16 * p.nt - 1) / (16 * p.nt);
     p.grid_y = (c.m + 16 * p.mt - 1) / (16 * p.mt);
@@ -413,15 +633,17 @@ static RowsPlan rows_plan(const RowsCall& c)
     const int per = (p.kt + p.nz - 1) / p.nz, rounds = (per + RW_MAX_WAVES - 1) / RW_MAX_WAVES;
     p.kw = (per + rounds - 1) / rounds;
     p.nc = (int)std::max<int64_t>(1, std::min<int64_t>(8 / p.kw, p.tiles * p.grid_y / device_cu_count()));
+    if (c.m > 16 * RW_MAX_MT) rows_plan_wide(c, p);
     p.grid_x = (p.tiles + p.nc - 1) / p.nc;
     const bool cvt = c.cb_dt != VQ2_DT_F16;
-    const int64_t units = p.nz > 1 ? p.grid_x * p.grid_y : 0;
+    const int64_t units = p.nz > 1 && !p.wide ? p.grid_x * p.grid_y : 0;
     p.e = up256((size_t)units * sizeof(uint32_t));
     p.a = p.e + up256((size_t)c.m * sizeof(int));
     p.h0 = p.a + (size_t)((c.m + 15) / 16) * p.kt * 512 * sizeof(half8_t);
     p.h1 = p.h0 + (cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
     p.part = p.h1 + (!cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
-    p.total = p.part + (size_t)units * p.nz * 256 * p.mt * p.nt * sizeof(float);
+    p.total = p.part + (p.wide && p.nz > 1 ? (size_t)p.nz * c.m * p.tiles * 16 : (size_t)units * p.nz * 256 * p.mt * p.nt) *
+                           sizeof(float);
     return p;
 }
 
@@ -469,6 +691,28 @@ static hipError_t rows_launch_s(int mt, const RowsArgs& a, dim3 grid, int waves,
     case 3: return rows_launch_t<S2, 3, 1>(a, grid, waves, st);
     default: return rows_launch_t<S2, 4, 1>(a, grid, waves, st);
     }
+}
+
+template <int S2, int MT, int TS>
+static hipError_t rows_wide_t(const RowsArgs& a, dim3 grid, hipStream_t st)
+{
+    // opt in to more than 64 KiB of dynamic LDS, once per instantiation
+    constexpr int SHM = 2 * MT * TS * 64 * (int)sizeof(half8_t);
+    static std::once_flag once;
+    static hipError_t attr = hipSuccess;
+    std::call_once(once, [] {
+        attr = hipFuncSetAttribute((const void*)rows_wide_kernel<S2, MT, TS>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, SHM);
+    });
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL((rows_wide_kernel<S2, MT, TS>), grid, dim3(64 * RW_WIDE_WAVES), SHM, st, a);
+    return hipGetLastError();
+}
+
+template <int S2>
+static hipError_t rows_wide_s(int mt, const RowsArgs& a, dim3 grid, hipStream_t st)
+{
+    return mt == 8 ? rows_wide_t<S2, 8, 4>(a, grid, st) : rows_wide_t<S2, 16, 2>(a, grid, st);
 }
 
 static hipError_t rows_pack_launch(const RowsPackArgs& p, hipStream_t st)
@@ -522,7 +766,7 @@ int rows_launch(const RowsCall& c)
     k.a = (half8_t*)(ws + p.a);
     k.e = (int*)(ws + p.e);
     k.cnt = (uint32_t*)ws;
-    k.n_cnt = p.nz > 1 ? (int)(p.grid_x * p.grid_y) : 0;
+    k.n_cnt = p.nz > 1 && !p.wide ? (int)(p.grid_x * p.grid_y) : 0;
     if (cvt) {
         k.cb0 = c.cb0;
         k.cb1 = c.cb1;
@@ -556,7 +800,22 @@ int rows_launch(const RowsCall& c)
         a.seg[a.nseg++] = RowsSeg{g.idx0, g.idx1, g.scale, g.y, g.y_stride, (int)g.rows, (int)tile};
         tile += (g.rows + 16 * p.nt - 1) / (16 * p.nt);
     }
+    a.tiles = (int)p.tiles;
     const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y, (unsigned)p.nz);
+    if (p.wide) {
+        switch (c.s2) {
+        case VQ2_S2_U8: err = rows_wide_s<VQ2_S2_U8>(p.mt, a, grid, st); break;
+        case VQ2_S2_U16: err = rows_wide_s<VQ2_S2_U16>(p.mt, a, grid, st); break;
+        default: err = rows_wide_s<VQ2_S2_NONE>(p.mt, a, grid, st); break;
+        }
+        if (err == hipSuccess && p.nz > 1) {
+            hipLaunchKernelGGL(rows_sum_kernel, dim3((unsigned)((p.tiles * 4 + 255) / 256), (unsigned)c.m), dim3(256), 0, st,
+                               a);
+            err = hipGetLastError();
+        }
+        if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm launch");
+        return VQ2_OK;
+    }
     switch (c.s2) {
     case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, a, grid, p.kw * p.nc, st); break;
     case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, a, grid, p.kw * p.nc, st); break;
