@@ -1,6 +1,8 @@
 """ctypes binding of libvq2_amd.so (the C ABI declared in include/vq2_amd.h).
 
-The library is built in-tree (``python -m compressai_amd.build`` or
+The library and ``_vq2_host`` (the native argument checks and launches of the
+entries that small calls spend their time in, csrc/vq2_host.cpp) are built
+in-tree (``python -m compressai_amd.build`` or
 ``__graft_entry__.build()``) and loaded from this package directory.  There is
 no fallback: if the library is missing, every entry raises.
 """
@@ -98,6 +100,7 @@ SIGNATURES = {
 }
 
 _lib = None
+_host = None
 
 
 class Vq2Error(RuntimeError):
@@ -154,6 +157,18 @@ def load():
         fn.restype = res
     _lib = L
     return _lib
+
+
+def host():
+    """The native host module, linked to the library (loaded once).  Raises
+    ImportError if it has not been built."""
+    global _host
+    if _host is None:
+        load()
+        from . import _vq2_host
+
+        _host = _vq2_host
+    return _host
 
 
 def check(status: int, what: str = "") -> None:

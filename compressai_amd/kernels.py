@@ -16,6 +16,11 @@ Additive entry points: vq_gemv_16_16 (4 bpw), batched GEMV (x of shape
 [B, n]), vq_rht, vq_swiglu_rht, vq_router_topk, vq_moe_down_combine,
 vq_gemv_argmax, vq_argmax, vq_dequant_rows, vq_decode_idx.
 
+The entries of the small calls (vq_sorted_gemv, vq_gemv_rht, vq_rows_gemm,
+vq_sorted_moe) hand the calls without given outputs to their native twins
+(csrc/vq2_host.cpp: the same checks and launch, ~8 us less host time each),
+which decline whatever the checks here have to look at.
+
 Every entry launches on the current torch stream of the input's device and
 raises ``Vq2Error`` (a RuntimeError) on any invalid argument.  There is no CPU
 or Triton fallback: CPU tensors are rejected and a missing library raises
@@ -27,6 +32,7 @@ is selectable (``out_dtype``; bf16 by default, as in the reference).
 from __future__ import annotations
 
 import ctypes
+import functools
 import weakref
 
 import torch
@@ -443,6 +449,10 @@ def vq_gemv_rht(x, mats, cb0, cb1, n, perm=None, sign=None, hb=2048, rht_scale=N
     (i0, i1 or None, scale, out_rows) sharing one cfg.  Returns the list of
     outputs ([out] or [B, out])."""
     n = int(n)
+    if ys is None and out_dtype is not None and hb and x.numel() <= FUSED_RHT_MAX_VALS:
+        ys = _lib.host().gemv_rht(x, mats, cb0, cb1, n, perm, sign, int(hb), rht_scale, rs, out_dtype)
+        if ys is not None:
+            return ys
     s2, mats = check_gemv_rht_mats(mats, cb0, cb1, n)
     dev = _dev(x, cb0, cb1, perm, sign, *[t for m in mats for t in m[:3]])
     x2 = _contig(x, "x").reshape(-1, n)
@@ -488,6 +498,10 @@ def vq_rows_gemm(x, mats, cb0, cb1, n, perm=None, sign=None, hb=2048, rht_scale=
     mats: list of (i0, i1 or None, scale, out_rows) sharing one cfg.  Returns
     the list of outputs [B, out_rows]."""
     n = int(n)
+    if ys is None and out_dtype is not None and act_dtype is not None:
+        ys = _lib.host().rows_gemm(x, mats, cb0, cb1, n, perm, sign, int(hb or 0), rht_scale, rs, act_dtype, out_dtype)
+        if ys is not None:
+            return ys
     s2, mats = check_gemv_rht_mats(mats, cb0, cb1, n)
     dev = _dev(x, cb0, cb1, perm, sign, *[t for m in mats for t in m[:3]])
     x2 = _contig(x, "x").reshape(-1, n)
@@ -679,6 +693,11 @@ def vq_sorted_gemv(x, mats, cb0, cb1, n, perm=None, sign=None, hb=2048, rht_scal
     last of them to finish sums their partials, in slice order, in the same
     launch.  Returns the list of outputs [out_rows]."""
     n = int(n)
+    if ys is None and slices is None and out_dtype is not None and x.is_cuda:
+        ys = _lib.host().sorted_gemv(x, mats, cb0, cb1, n, perm, sign, int(hb or 0), rht_scale, rs, out_dtype,
+                                     _cu_count(x.device), _workspace)
+        if ys is not None:
+            return ys
     planes = [m[0] for m in mats]
     if not 1 <= len(mats) <= 4 or any(p.n != n for p in planes):
         raise Vq2Error("vq_sorted_gemv: 1..4 matrices of width n")
@@ -925,6 +944,7 @@ _MOE_RATE = 1460.0
 _MOE_FIXED_US = (2.5, 2.0)
 
 
+@functools.lru_cache(maxsize=512)
 def moe_slices(units, codes_per_unit, cu, fixed_us, one_launch=False):
     """Slices per chunk for `units` (pair, chunk) units: the count that
     minimises rounds x (work per slice + fixed cost), with one 16-wave
@@ -946,6 +966,17 @@ def moe_slices(units, codes_per_unit, cu, fixed_us, one_launch=False):
         if best_t is None or t < best_t - 1e-9:
             best, best_t = s, t
     return best
+
+
+def _moe_launch_slices(T, P, gate_up, down, dev, H, I, hb_h, hb_i):
+    """(gate_up, down) slices per chunk of one vq_sorted_moe call."""
+    cu = _cu_count(dev)
+    # the library runs gate_up and down as one launch for these shapes
+    # (2048-point and 512-point rotations, at most 128 pairs)
+    one = H == 2048 and I == 512 and hb_h == 2048 and hb_i == 512 and T * P <= 127
+    st = 2 if gate_up.has_stage2 else 1
+    return (moe_slices(T * P * gate_up.chunks, st * gate_up.rows_per_chunk * gate_up.ng, cu, _MOE_FIXED_US[0], one),
+            moe_slices(T * P * down.chunks, st * down.rows_per_chunk * down.ng, cu, _MOE_FIXED_US[1], one))
 
 
 def _rot_tables(rot, n, what):
@@ -972,6 +1003,11 @@ def vq_sorted_moe(h, gate_up: SortedPool, gu_scale, down: SortedPool, dn_scale, 
     (out, ids int32 [T, top_k + 1], w fp32 [T, top_k + 1]).  rot_h / rot_i:
     (perm int32, sign int8, hb, scale).  Two-stage pools (the (16,8) 3 bpw
     experts) take their stage-2 codebook cb1 ([256, 8] in cb's dtype)."""
+    if out is None and slices is None and cb1 is None and out_dtype is not None and h.is_cuda:
+        r = _lib.host().sorted_moe(h, gate_up, gu_scale, down, dn_scale, cb, rot_h, rot_i, ids, w, logits, top_k, shared_id,
+                                   shared_gate, out_dtype, _moe_launch_slices, _workspace)
+        if r is not None:
+            return r
     H = gate_up.ng * 8
     I = down.ng * 8
     if gate_up.rows != 2 * I or down.rows != H or gate_up.n_experts != down.n_experts:
@@ -1012,13 +1048,7 @@ def vq_sorted_moe(h, gate_up: SortedPool, gu_scale, down: SortedPool, dn_scale, 
     elif out.numel() != T * H or not out.is_contiguous():
         raise Vq2Error(f"out must be a contiguous [{T}, {H}]")
     if slices is None:
-        cu = _cu_count(dev)
-        # the library runs gate_up and down as one launch for these shapes
-        # (2048-point and 512-point rotations, at most 128 pairs)
-        one = H == 2048 and I == 512 and int(rot_h[2]) == 2048 and int(rot_i[2]) == 512 and T * P <= 127
-        st = 2 if gate_up.has_stage2 else 1
-        sg = moe_slices(T * P * gate_up.chunks, st * gate_up.rows_per_chunk * gate_up.ng, cu, _MOE_FIXED_US[0], one)
-        sd = moe_slices(T * P * down.chunks, st * down.rows_per_chunk * down.ng, cu, _MOE_FIXED_US[1], one)
+        sg, sd = _moe_launch_slices(T, P, gate_up, down, dev, H, I, int(rot_h[2]), int(rot_i[2]))
     else:
         sg, sd = (int(v) for v in slices)
     lib = _lib.load()

@@ -272,14 +272,14 @@ class PackedProjections(nn.Module):
                 self.sorted.append(sp)
 
     def forward(self, x, out_dtype=None):
-        lins = self.lins
+        lins = list(self.lins)
         a = lins[0]
         x2 = x.reshape(-1, a.n).contiguous()
         i0, i1, cb0, cb1 = a._planes()
         od = out_dtype or x.dtype
         B = x2.shape[0]
-        rows = (_rows_ok(x2, a.n, a.rot) and not any(m.planes_released for m in lins)
-                and all(m.act_dtype == a.act_dtype for m in lins))
+        rows = (_rows_ok(x2, a.n, a.rot)
+                and all(not m.planes_released and m.act_dtype == a.act_dtype for m in lins))
         if self.sorted is not None and B == 1 and cb0.dtype in (torch.float16, torch.bfloat16):
             xs, perm, sign, hb, sc = a._sorted_args(x2.reshape(-1))
             ys = K.vq_sorted_gemv(xs, [(sp, m.scale) for sp, m in zip(self.sorted, lins)], cb0, cb1, a.n, perm,

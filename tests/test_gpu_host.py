@@ -1,0 +1,109 @@
+"""The native twins of the small calls' entries (csrc/vq2_host.cpp) against
+the Python entries they stand in for: the same launch, so bit-identical results
+(given outputs take the Python entry), over types, strides of the batch and
+one to four matrices; calls they decline raise what the Python entry raises;
+each stream has its own workspace."""
+import pytest
+import torch
+
+from compressai_amd import _lib, kernels as K, synth
+from compressai_amd.kernels import Vq2Error
+from compressai_amd.moe import ResidentMoEExperts
+
+pytestmark = pytest.mark.gpu
+
+
+def _mats(dev, seed, n, rows, bpw):
+    ms = [synth.vq_matrix(seed + i, r, n, bpw=bpw) for i, r in enumerate(rows)]
+    cb0 = synth.codebook(seed + 50).to(dev)
+    cb1 = {2: None, 3: synth.codebook(seed + 51, rows=256), 4: synth.codebook(seed + 51)}[bpw]
+    return ms, cb0, None if cb1 is None else cb1.to(dev)
+
+
+def _tables(dev, n):
+    return synth.permutation(8810, n).to(dev), synth.signs(8811, n).to(dev)
+
+
+@pytest.mark.parametrize("n,rows,bpw,x_dtype,y_dtype", [
+    (2048, (2048,), 2, torch.float16, torch.float16),           # one slice
+    (2048, (6144, 6144), 4, torch.bfloat16, torch.bfloat16),    # slices: the stream's workspace
+    (512, (96, 17, 1, 33), 3, torch.float32, torch.float32),
+])
+def test_sorted_gemv(dev, n, rows, bpw, x_dtype, y_dtype):
+    ms, cb0, cb1 = _mats(dev, 8800, n, rows, bpw)
+    mats = [(K.SortedPlanes(m["idx0"], m["idx1"], r, n, device=dev), m["scale"].to(dev)) for m, r in zip(ms, rows)]
+    perm, sign = _tables(dev, n)
+    x = synth.activations(8820, n, dtype=x_dtype).to(dev)
+    for kw in (dict(hb=min(n, 2048)), dict(hb=0, rs=0.5), dict(hb=64, rht_scale=0.25)):
+        p, s = (perm, sign) if kw["hb"] else (None, None)
+        ref = K.vq_sorted_gemv(x, mats, cb0, cb1, n, p, s, ys=[torch.empty(r, dtype=y_dtype, device=dev) for r in rows], **kw)
+        side = torch.cuda.Stream(dev)
+        side.wait_stream(torch.cuda.current_stream(dev))
+        with torch.cuda.stream(side):
+            got = K.vq_sorted_gemv(x, mats, cb0, cb1, n, p, s, out_dtype=y_dtype, **kw)
+        torch.cuda.synchronize(dev)
+        assert len(got) == len(ref) and all(torch.equal(a, b) and a.dtype == y_dtype for a, b in zip(got, ref))
+
+
+@pytest.mark.parametrize("fn,B", [("vq_gemv_rht", 1), ("vq_gemv_rht", 2), ("vq_rows_gemm", 3), ("vq_rows_gemm", 70)])
+@pytest.mark.parametrize("bpw", [2, 3, 4])
+def test_rotated_products(dev, fn, B, bpw):
+    n, rows = 1024, (300, 77)
+    ms, cb0, cb1 = _mats(dev, 8830, n, rows, bpw)
+    mats = [(m["idx0"].to(dev), None if m["idx1"] is None else m["idx1"].to(dev), m["scale"].to(dev), r)
+            for m, r in zip(ms, rows)]
+    perm, sign = _tables(dev, n)
+    x = synth.activations(8840, (B, n), dtype=torch.bfloat16).to(dev)
+    call = getattr(K, fn)
+    got = call(x, mats, cb0, cb1, n, perm, sign, 1024, out_dtype=torch.bfloat16)
+    ref = call(x, mats, cb0, cb1, n, perm, sign, 1024,
+               ys=[torch.empty(B, r, dtype=torch.bfloat16, device=dev) for r in rows])
+    assert all(torch.equal(a, b) and a.shape == b.shape for a, b in zip(got, ref))
+
+
+@pytest.mark.parametrize("T", [1, 5, 20])
+def test_sorted_moe(dev, T):
+    E, P = 12, 3
+    gu, dn = synth.indices16(8850, (E, 1024, 256)).to(dev), synth.indices16(8851, (E, 2048, 64)).to(dev)
+    gus, dns = synth.scales(8852, (E, 1024)).to(dev), synth.scales(8853, (E, 2048)).to(dev)
+    mod = ResidentMoEExperts.from_pools(gu, gus, dn, dns, synth.codebook(8854).to(dev), sorted_layout=True)
+    h = synth.activations(8855, (T, 2048)).to(dev)
+    ids = torch.randint(0, E, (T, P), generator=synth.gen(8856)).to(dev)
+    w = torch.rand(T, P, generator=synth.gen(8857)).to(dev)
+    rh, ri = mod._rots()
+    args = (h, mod.sorted_gu, gus, mod.sorted_dn, dns, mod.cb16, rh, ri)
+    ref = K.vq_sorted_moe(*args, ids=ids, w=w, out=torch.empty(T, 2048, device=dev))
+    assert torch.equal(K.vq_sorted_moe(*args, ids=ids, w=w), ref)
+    lg = synth.activations(8858, (T, E - 1), dtype=torch.float32).to(dev)
+    kw = dict(logits=lg, top_k=2, shared_id=E - 1, shared_gate=synth.activations(8859, 2048).to(dev))
+    ref = K.vq_sorted_moe(*args, out=torch.empty(T, 2048, device=dev), **kw)
+    assert all(torch.equal(a, b) for a, b in zip(K.vq_sorted_moe(*args, **kw), ref))
+
+
+def test_declined_calls(dev):
+    """What the native checks decline, the Python entry refuses or handles."""
+    n = 512
+    ms, cb0, _ = _mats(dev, 8870, n, (64,), 2)
+    i0, sc = ms[0]["idx0"].to(dev), ms[0]["scale"].to(dev)
+    x = torch.zeros(2, n, dtype=torch.float16, device=dev)
+    sp = K.SortedPlanes(ms[0]["idx0"], None, 64, n, device=dev)
+    host = _lib.host()
+    bad = [dict(x=x.cpu()), dict(x=x[:, ::2]), dict(cb0=cb0[:100]), dict(perm=torch.zeros(n, dtype=torch.int64, device=dev)),
+           dict(mats=[(i0, None, sc[:3], 64)]), dict(mats=[(i0, None, sc.cpu(), 64)]), dict(mats=[])]
+    for b in bad:
+        a = dict(x=x, mats=[(i0, None, sc, 64)], cb0=cb0, perm=None)
+        a.update(b)
+        args = (a["x"], a["mats"], a["cb0"], None, n, a["perm"], None, n)
+        assert host.gemv_rht(*args, None, 1.0, torch.float32) is None, b
+        assert host.rows_gemm(*args, None, 1.0, torch.float32, torch.float32) is None, b
+        with pytest.raises(Vq2Error):
+            K.vq_gemv_rht(*args)
+        with pytest.raises(Vq2Error):
+            K.vq_rows_gemm(*args)
+    with pytest.raises(Vq2Error):
+        K.vq_sorted_gemv(x[0], [(sp, sc)], cb0.float(), None, n, hb=0)
+    with pytest.raises(Vq2Error):
+        K.vq_sorted_gemv(x, [(sp, sc)], cb0, None, n, hb=0)
+    # uint16 planes: handled by the Python entry
+    (y,) = K.vq_gemv_rht(x, [(i0.view(torch.uint16), None, sc, 64)], cb0, None, n, hb=n)
+    assert torch.equal(y, K.vq_gemv_rht(x, [(i0, None, sc, 64)], cb0, None, n, hb=n)[0])
