@@ -34,8 +34,9 @@
 // 7e-7.
 //
 // Measured (35B shape, us a layer, router included, one-pair kernels before):
-// 72 tokens 521 -> 493, 128 tokens 896 -> 509, 512 tokens 3526 -> 609; at 512
-// tokens gate_up gathers 67 M codes in 0.37 ms, down 34 M in 0.2.
+// 72 tokens 521 -> 493, 128 tokens 896 -> 509, 512 tokens 3526 -> 590; at 512
+// tokens gate_up gathers 67 M codes in 0.37 ms, down 34 M in 0.2 (with all
+// codes alike 0.17 and 0.12).
 #include <algorithm>
 #include <mutex>
 
@@ -163,9 +164,23 @@ __device__ void moe_plan(const MoePlanArgs& p, int* s_cnt)
     const int T = (int)blockDim.x, tid = threadIdx.x, E = p.n_experts;
     for (int i = tid; i < E; i += T) s_cnt[i] = 0;
     __syncthreads();
-    for (int i = tid; i < p.pairs; i += T) {
-        const int64_t e = moe_pair_id(p, i);
-        if (e >= 0 && e < E) atomicAdd(&s_cnt[e], 1);
+    // ids in batches, so that their loads are in flight together; one batch
+    // (up to 5120 pairs with 256 threads) stays in registers for both passes
+    // (one load at a time the two passes over 4608 pairs took ~12 us)
+    constexpr int NB = 20;
+    int e[NB];
+    auto load_ids = [&](int i0) {
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int64_t id = moe_pair_id(p, min(i0 + j * T, p.pairs - 1));
+            e[j] = i0 + j * T < p.pairs && id >= 0 && id < E ? (int)id : -1;
+        }
+    };
+    for (int i0 = tid; i0 - tid < p.pairs; i0 += NB * T) {
+        load_ids(i0);
+#pragma unroll
+        for (int j = 0; j < NB; j++)
+            if (e[j] >= 0) atomicAdd(&s_cnt[e[j]], 1);
     }
     __syncthreads();
     // thread t scans the experts [t * per, t * per + per)
@@ -198,15 +213,20 @@ __device__ void moe_plan(const MoePlanArgs& p, int* s_cnt)
         if (tid == MR_PLAN_T - 1) *p.n_tiles = s_sum[1][tid];
     }
     __syncthreads();
-    for (int i = tid; i < p.pairs; i += T) {
-        const int64_t e = moe_pair_id(p, i);
-        int slot = -1;
-        if (e >= 0 && e < E) {
-            slot = atomicAdd(&s_cnt[e], 1);
-            p.slot_tok[slot] = i / p.P;
-            p.slot_pair[slot] = i;
+    for (int i0 = tid; i0 - tid < p.pairs; i0 += NB * T) {
+        if (p.pairs > NB * T) load_ids(i0);
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            const int i = i0 + j * T;
+            if (i >= p.pairs) break;
+            int slot = -1;
+            if (e[j] >= 0) {
+                slot = atomicAdd(&s_cnt[e[j]], 1);
+                p.slot_tok[slot] = i / p.P;
+                p.slot_pair[slot] = i;
+            }
+            p.pair_slot[i] = slot;
         }
-        p.pair_slot[i] = slot;
     }
 }
 
@@ -424,15 +444,16 @@ __global__ void __launch_bounds__(256) moe_rows_combine_kernel(const float* shar
     const int t = blockIdx.y, c = (int)blockIdx.x * 256 + threadIdx.x;
     if (c * 4 >= H) return;
     f32x4_t sum = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (int k0 = 0; k0 < P; k0 += 8) {
-        f32x4_t v[8];
-        int slot[8];
+    constexpr int NB = 12;  // pairs whose loads are in flight together
+    for (int k0 = 0; k0 < P; k0 += NB) {
+        f32x4_t v[NB];
+        int slot[NB];
 #pragma unroll
-        for (int k = 0; k < 8; k++) slot[k] = pair_slot[(int64_t)t * P + min(k0 + k, P - 1)];
+        for (int k = 0; k < NB; k++) slot[k] = pair_slot[(int64_t)t * P + min(k0 + k, P - 1)];
 #pragma unroll
-        for (int k = 0; k < 8; k++) v[k] = *((const f32x4_t*)(share + (int64_t)max(slot[k], 0) * H) + c);
+        for (int k = 0; k < NB; k++) v[k] = *((const f32x4_t*)(share + (int64_t)max(slot[k], 0) * H) + c);
 #pragma unroll
-        for (int k = 0; k < 8; k++) {
+        for (int k = 0; k < NB; k++) {
             if (k0 + k >= P) continue;
             const float bad = __builtin_nanf("");
             sum += slot[k] >= 0 ? v[k] : f32x4_t{bad, bad, bad, bad};
