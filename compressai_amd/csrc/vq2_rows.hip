@@ -22,13 +22,14 @@
 // sum; here the activation is converted once, a wave reads its operand
 // fragments as whole 1 KiB lines straight into registers, and the K split
 // lies inside the workgroup (waves take k tiles in turn and their sums meet
-// in LDS), so nothing is written but y.  Measured (graph replays, us a call,
-// rotation included; before: vq2_rht, vq2_gemm_small_m per 64 rows and its
-// reduce launch): 2048 x 6144 at 4 bpw, 16 rows 29.3 -> 27.5; 6144 x 2048 at
-// 4 bpw, 64 rows 37.1 -> 31.2; two 6144 x 2048 at 3 bpw, 64 rows, bf16
-// 64.2 -> 38.6; 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5, 1024 rows
-// 264.8 -> 50.4; two 6144 x 2048 at 4 bpw, 1024 rows 981 -> 192.  Bound by the gathers (13 us of the 4 bpw calls) and, below
-// about a million codes, by the two launches' latency (~12 us).
+// in LDS), so nothing is written but y.  Measured, us a call, rotation
+// included (before: vq2_rht, vq2_gemm_small_m per 64 rows and its reduce
+// launch): 2048 x 6144 at 4 bpw, 16 rows 34.0 -> 25.7; two 6144 x 2048 at
+// 3 bpw, 64 rows, bf16 75.2 -> 31.5; 2048 x 2048 at 2 bpw, 100 rows 52.0 ->
+// 33.1; two 6144 x 2048 at 4 bpw, 1024 rows 979 -> 174; in graph replays
+// 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5.  Bound by the gathers (13 us
+// of a 6144 x 2048 call at 4 bpw) and, below about a million codes, by the
+// two launches' latency (~12 us).
 //
 // Fragment layout: v_mfma_f32_16x16x32_f16 takes 8 consecutive k of row
 // l % 16 from lane l, k block l / 16.  A k tile is 32 groups (256 k); its
@@ -196,7 +197,8 @@ struct RowsArgs {
     float rs;
     int nseg;
     int kw;  // waves of a workgroup that share a column tile's k tiles
-    int nz;  // workgroups that share them (gridDim.z); nc is 1 then
+    int nc;  // column tiles of a workgroup of rows_gemm_kernel
+    int nz;  // workgroups that share a tile's k tiles (gridDim.z); nc is 1 then
     float* part;    // nz > 1: [row block][column tile][nz][16 MT][16 NT] sums
     uint32_t* cnt;  // nz > 1: arrivals per [row block][column tile], zero
     int tiles;      // column tiles of all matrices
@@ -247,20 +249,25 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     touch_kernargs(a);
     extern __shared__ __align__(16) float s_red[];  // [waves][16 MT][16 NT + 1]
     __shared__ half8_t s_c1[S2 == VQ2_S2_U8 ? 256 : 1];
+    __shared__ int s_e[16 * MT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nl = lane & 15, q = lane >> 4;
-    const int kw = a.kw, nc = (int)(blockDim.x >> 6) / kw;
-    const int tile = (int)blockIdx.x * nc + wave / kw;
-    const int k0 = (int)blockIdx.z * kw + wave % kw, kstep = kw * a.nz;
+    const int kw = a.kw, nc = a.nc;
+    const int ct0 = nc == 1 ? 0 : wave / kw;  // this wave's column tile of the workgroup
+    const int tile = (int)blockIdx.x * nc + ct0;
+    const int k0 = (int)blockIdx.z * kw + wave - ct0 * kw, kstep = kw * a.nz;
     const RowsSeg& sg = rows_seg(a, tile);
     const int col0 = (tile - sg.tile0) * 16 * NT;  // may lie past the last matrix's rows (tail workgroup)
     const int mt0 = (int)blockIdx.y * MT;
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
-    if constexpr (S2 == VQ2_S2_U8) {
-        for (int i = tid; i < 256; i += (int)blockDim.x) s_c1[i] = a.cb1[i];
-        __syncthreads();
-    }
+    // what the epilogue needs, loaded ahead of everything else: the rows'
+    // exponents and (one column tile: a thread keeps its column) the scale.
+    // Finding the matrix of each output again, with its divisions and its
+    // loads, took 4.4 of 35.9 us for gate and up of 6144 x 2048 at 3 bpw and 64 rows.
+    const int e_pre = tid < 16 * MT ? a.e[min(mt0 * 16 + tid, a.m - 1)] : 0;
+    const int ecol = min(col0 + tid % (16 * NT), sg.rows - 1);
+    const uint32_t s_pre = nc == 1 ? load_raw(sg.scale, a.s_dt, ecol) : 0u;
 
     int64_t rowoff[NT];
 #pragma unroll
@@ -288,6 +295,10 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         for (int c = 0; c < NT; c++) cd[c].load(sg, rowoff[c] + (g < a.ng ? g : 0));
     };
     if (k0 < a.kt) load_codes(k0);
+    if constexpr (S2 == VQ2_S2_U8) {
+        for (int i = tid; i < 256; i += (int)blockDim.x) s_c1[i] = a.cb1[i];
+        __syncthreads();
+    }
     for (int kt = k0; kt < a.kt; kt += kstep) {
         const bool g_ok = kt * RW_TILE_G + q * 8 < a.ng;
         half8_t b0[8][NT], b1[8][NT];
@@ -331,6 +342,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         for (int c = 0; c < NT; c++)
 #pragma unroll
             for (int e = 0; e < 4; e++) mine[(i * 16 + q * 4 + e) * LD + c * 16 + nl] = acc[i][c][e];
+    if (tid < 16 * MT) s_e[tid] = e_pre;
     __syncthreads();
     const int mrows = min(16 * MT, a.m - mt0 * 16);
     const float* red = s_red;
@@ -360,6 +372,19 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         __syncthreads();
         nred = 1;
     }
+    if (nc == 1) {
+        // (blockDim is a multiple of 16 NT: the thread's column stays)
+        const int c = tid % (16 * NT);
+        const float s = raw_as_f32(s_pre, a.s_dt);
+        if (col0 + c >= sg.rows) return;
+        for (int r = tid / (16 * NT); r < mrows; r += (int)blockDim.x / (16 * NT)) {
+            const float* p = red + r * LD + c;
+            float sum = 0.0f;
+            for (int w = 0; w < nred; w++) sum += p[w * TILE];
+            store_from_f32(sg.y, a.y_dt, (int64_t)(mt0 * 16 + r) * sg.y_stride + col0 + c, (ldexpf(sum, -s_e[r]) * s) * a.rs);
+        }
+        return;
+    }
     for (int t = tid; t < nc * mrows * 16 * NT; t += (int)blockDim.x) {
         const int c = t % (16 * NT), u = t / (16 * NT);
         const int r = u % mrows, ct = u / mrows;
@@ -370,9 +395,8 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         const float* p = red + ct * kw * TILE + r * LD + c;
         float sum = 0.0f;
         for (int w = 0; w < nred; w++) sum += p[w * TILE];
-        const int row = mt0 * 16 + r;
         const float s = load_as_f32(so.scale, a.s_dt, col);
-        store_from_f32(so.y, a.y_dt, (int64_t)row * so.y_stride + col, (ldexpf(sum, -a.e[row]) * s) * a.rs);
+        store_from_f32(so.y, a.y_dt, (int64_t)(mt0 * 16 + r) * so.y_stride + col, (ldexpf(sum, -s_e[r]) * s) * a.rs);
     }
 }
 
@@ -790,6 +814,7 @@ int rows_launch(const RowsCall& c)
     a.y_dt = c.y_dt;
     a.rs = c.rs;
     a.kw = p.kw;
+    a.nc = p.nc;
     a.nz = p.nz;
     a.part = (float*)(ws + p.part);
     a.cnt = k.cnt;
