@@ -25,7 +25,7 @@
 // in LDS), so nothing is written but y.  Measured, us a call, rotation
 // included (before: vq2_rht, vq2_gemm_small_m per 64 rows and its reduce
 // launch): 2048 x 6144 at 4 bpw, 16 rows 34.0 -> 25.7; two 6144 x 2048 at
-// 3 bpw, 64 rows, bf16 75.2 -> 31.5; 2048 x 2048 at 2 bpw, 100 rows 52.0 ->
+// 3 bpw, 64 rows, bf16 75.2 -> 31.5; 2999 x 4096 at 2 bpw, 100 rows 52.0 ->
 // 33.1; two 6144 x 2048 at 4 bpw, 1024 rows 979 -> 174; in graph replays
 // 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5.  Bound by the gathers (13 us
 // of a 6144 x 2048 call at 4 bpw) and, below about a million codes, by the
@@ -407,8 +407,9 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
 // gathered once per 128 or 256 rows instead of 64.  Bound by those gathers and,
 // as a wave reads every operand of the rows from LDS for its 16 columns, by
 // the LDS rate (with all codes alike, two 6144 x 2048 matrices at 4 bpw and
-// 1024 rows take 133 of 192 us).  Measured there, us a call: 8 waves and 4
-// steps a stage 208, 8 and 2 205, 4 and 2 192; 32 columns a wave, which halves
+// 1024 rows took 133 us of the 192 of a graph replay; 173 a call now).
+// Measured there, us a replay: 8 waves and 4 steps a stage 208, 8 and 2 205,
+// 4 and 2 192; 32 columns a wave, which halves
 // the LDS reads, spills at 256 rows (266), and so do 512 rows (216).
 template <int S2, int MT, int TS>
 __global__ void __launch_bounds__(64 * RW_WIDE_WAVES, 2) rows_wide_kernel(const RowsArgs a)
