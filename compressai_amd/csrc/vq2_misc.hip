@@ -143,7 +143,7 @@ int router_launch(const void* logits, int l_dt, int64_t tokens, int64_t n_expert
     if (tokens == 0) return VQ2_OK;
     if (n_experts <= 0 || n_experts > ROUTER_MAX_E)
         return set_error(VQ2_ERR_UNSUPPORTED, "vq2 router: n_experts=%lld not in [1, %d]", (long long)n_experts, ROUTER_MAX_E);
-    if (k <= 0 || k > 32 || k > n_experts) return set_error(VQ2_ERR_ARG, "vq2 router: k=%d out of range", k);
+    if (k <= 0 || k > VQ2_ROUTER_MAX_TOPK || k > n_experts) return set_error(VQ2_ERR_ARG, "vq2 router: k=%d out of range", k);
     if (tokens > 0x7FFFFFFF) return set_error(VQ2_ERR_UNSUPPORTED, "vq2 router: too many tokens");
     hipLaunchKernelGGL(router_kernel, dim3((unsigned)tokens), dim3(64), 0, (hipStream_t)stream, logits, l_dt,
                        n_experts, k, h, h_dt, hidden, gate, g_dt, shared_id, ids, w);

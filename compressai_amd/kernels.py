@@ -1072,6 +1072,8 @@ def vq_sorted_moe(h, gate_up: SortedPool, gu_scale, down: SortedPool, dn_scale, 
 MOE_ROWS_MAX_EXPERTS = 4096
 MOE_ROWS_MAX_TOKENS = 65535
 MOE_ROWS_MIN_PAIRS = 256
+# Experts a token vq_router_topk selects at most (VQ2_ROUTER_MAX_TOPK of the header).
+ROUTER_MAX_TOPK = 32
 
 
 def moe_rows_faster(pairs, n_experts, hidden, inter) -> bool:

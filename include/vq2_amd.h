@@ -315,7 +315,8 @@ int vq2_swiglu_rht(const void* gu, int gu_dt, int64_t gu_stride, int64_t inter,
  * If shared_id >= 0, slot k of each row gets the shared expert:
  *   ids[t, k] = shared_id,  w[t, k] = sigmoid(sum_i gate[i] * h[t, i])
  * (Qwen3_5MoeSparseMoeBlock.forward shared-expert gate), with h [tokens, hidden].
- * n_experts <= 1024, k <= 32. */
+ * n_experts <= 1024, k <= VQ2_ROUTER_MAX_TOPK. */
+#define VQ2_ROUTER_MAX_TOPK 32
 int vq2_router_topk(const void* logits, int l_dt, int64_t tokens, int64_t n_experts, int k,
                     const void* h, int h_dt, int64_t hidden, const void* gate, int g_dt, int64_t shared_id,
                     int32_t* ids, float* w, void* stream);

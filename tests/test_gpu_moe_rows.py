@@ -137,3 +137,20 @@ def test_layer_takes_the_grouped_path_and_keeps_its_precision(dev, cb_dtype):
     one = layer(h, lg)
     norm = lambda a: np.linalg.norm(a.double().cpu().numpy() - ref) / np.linalg.norm(ref)
     assert norm(out) <= 1.02 * norm(one), (norm(out), norm(one))
+
+
+def test_layer_with_a_top_k_above_the_router_entrys_runs_for_any_token_count(dev):
+    """Forty experts a token: more than vq_router_topk selects, so a chunk
+    that would be grouped stays on the one-pair kernels and its router, and
+    gives each token what a call of few tokens gives it."""
+    E, k, T = 64, 40, 40
+    gu, gus, dn, dns = _pools(9890, E + 1, 512, 64)
+    layer = MoELayer(gu.to(dev), (gus.float() * 512 ** -0.5).half().to(dev), dn.to(dev),
+                     (dns.float() * 64 ** -0.5).half().to(dev), synth.codebook(9895).to(dev),
+                     synth.activations(9896, 512).to(dev) * 0.02, top_k=k)
+    assert K.moe_rows_faster(T * (k + 1), E + 1, 512, 64)
+    h = synth.activations(9897, (T, 512)).to(dev)
+    lg = synth.activations(9898, (T, E), dtype=torch.float32).to(dev)
+    out = layer(h, lg)
+    few = torch.cat([layer(h[t:t + 4], lg[t:t + 4]) for t in range(0, T, 4)])
+    assert float((out - few).abs().max()) <= TOL * float(few.abs().max())

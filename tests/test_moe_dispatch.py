@@ -1,0 +1,56 @@
+"""Which entry a sorted MoE module calls (on the CPU, the entries replaced by
+recorders): the grouped kernel takes no call that it, or the router in front
+of it, refuses and the one-pair kernels take, and none that those refuse."""
+import re
+
+import pytest
+import torch
+
+from compressai_amd import _lib, kernels as K, synth
+from compressai_amd.moe import MoELayer
+
+E, H, I = 65, 64, 64
+
+
+@pytest.fixture
+def calls(monkeypatch):
+    """Names of the expert entries called, in order; their results are zeros."""
+    names = []
+
+    def moe_rows(h, ids, w, *a, **kw):
+        names.append("rows")
+        return torch.zeros(h.reshape(-1, H).shape)
+
+    def sorted_moe(h, *a, logits=None, **kw):
+        names.append("sorted")
+        out = torch.zeros(h.reshape(-1, H).shape)
+        return out if logits is None else (out, None, None)
+
+    def router(logits, k, *a, **kw):
+        T = logits.shape[0]
+        return torch.zeros(T, k + 1, dtype=torch.int32), torch.zeros(T, k + 1)
+
+    monkeypatch.setattr(K, "vq_moe_rows", moe_rows)
+    monkeypatch.setattr(K, "vq_sorted_moe", sorted_moe)
+    monkeypatch.setattr(K, "vq_router_topk", router)
+    return names
+
+
+def _layer(top_k):
+    gu, dn = synth.indices16(8620, (E, 2 * I, H // 8)), synth.indices16(8621, (E, H, I // 8))
+    return MoELayer(gu, synth.scales(8622, (E, 2 * I)), dn, synth.scales(8623, (E, H)), synth.codebook(8624),
+                    torch.zeros(H), top_k=top_k, sorted_layout=True)
+
+
+@pytest.mark.parametrize("top_k,entry", [(8, "rows"), (32, "rows"), (33, "sorted"), (64, "sorted")])
+def test_top_k_of_the_router_in_front_of_the_grouped_kernel(calls, top_k, entry):
+    """The router entry takes VQ2_ROUTER_MAX_TOPK experts a token, the one
+    built into the one-pair launch 64: layers above stay there for any T."""
+    limit = int(re.search(r"#define VQ2_ROUTER_MAX_TOPK (\d+)", _lib.HEADER_PATH.read_text()).group(1))
+    assert limit == K.ROUTER_MAX_TOPK and (entry == "rows") == (top_k <= limit)
+    layer = _layer(top_k)
+    T = 12000 // (top_k + 1)
+    assert K.moe_rows_faster(T * (top_k + 1), E, H, I)
+    layer(torch.zeros(1, H), torch.zeros(1, E - 1))
+    layer(torch.zeros(T, H), torch.zeros(T, E - 1))
+    assert calls == ["sorted", entry]
