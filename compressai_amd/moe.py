@@ -269,7 +269,8 @@ class MoELayer(nn.Module):
         if m.sorted_gu is not None and self.n_routed <= 256:
             # (calls that the sorted path refuses are left to it, and those
             # whose top_k only its built-in router takes)
-            if (self.n_routed < m.num_experts and router_logits.numel() <= 256 * T and self.top_k <= K.ROUTER_MAX_TOPK
+            if (self.n_routed < m.num_experts and self.top_k <= K.ROUTER_MAX_TOPK
+                    and self.top_k * T <= router_logits.numel() <= min(256, m.num_experts) * T
                     and m._rows_ok(h2, T * (self.top_k + 1))):
                 return m._rows(h2, *self.route(h2, router_logits.reshape(T, -1)))
             rh, ri = m._rots()

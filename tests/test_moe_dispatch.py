@@ -54,3 +54,14 @@ def test_top_k_of_the_router_in_front_of_the_grouped_kernel(calls, top_k, entry)
     layer(torch.zeros(1, H), torch.zeros(1, E - 1))
     layer(torch.zeros(T, H), torch.zeros(T, E - 1))
     assert calls == ["sorted", entry]
+
+
+@pytest.mark.parametrize("columns,entry", [(E - 1, "rows"), (E, "rows"), (E + 1, "sorted"), (7, "sorted")])
+def test_logits_the_one_pair_launch_refuses_are_left_to_it(calls, columns, entry):
+    """Logits of more columns than the pool has entries, or fewer than top_k:
+    refused for few tokens, so for many as well."""
+    T = 1500
+    layer = _layer(8)
+    assert K.moe_rows_faster(T * 9, E, H, I)
+    layer(torch.zeros(T, H), torch.zeros(T, columns))
+    assert calls == [entry]
