@@ -175,11 +175,11 @@ class ResidentMoEExperts(nn.Module):
         return (rh._perm32, rh._sign8, rh.hb, rh.scale), (ri._perm32, ri._sign8, ri.hb, ri.scale)
 
     def _rows_ok(self, h, pairs):
-        """Whether h [T, H] with that many pairs takes kernels.vq_moe_rows:
+        """Whether h [..., H] with that many pairs takes kernels.vq_moe_rows:
         enough pairs to share the experts' codes, the reference pools there
         in the form it reads, and what the sorted path takes besides."""
         gu, dn = self.gate_up_idx, self.down_idx
-        return (gu is not None and h.shape[0] <= K.MOE_ROWS_MAX_TOKENS
+        return (gu is not None and h.numel() // self.hidden_dim <= K.MOE_ROWS_MAX_TOKENS
                 and self.num_experts <= K.MOE_ROWS_MAX_EXPERTS and max(self.hidden_dim, self.intermediate_dim) <= 8192
                 and min(self.rot_h.hb, self.rot_i.hb) >= 64 and gu.is_contiguous() and dn.is_contiguous()
                 and all(t.data_ptr() % 16 == 0 for t in (gu, dn, h))

@@ -65,3 +65,15 @@ def test_logits_the_one_pair_launch_refuses_are_left_to_it(calls, columns, entry
     assert K.moe_rows_faster(T * 9, E, H, I)
     layer(torch.zeros(T, H), torch.zeros(T, columns))
     assert calls == [entry]
+
+
+def test_token_count_of_activations_with_more_dims(calls):
+    """experts() flattens h: the grouped kernel's token limit counts tokens,
+    whatever the first dimension holds."""
+    m = _layer(1).experts_mod
+    T = K.MOE_ROWS_MAX_TOKENS + 1
+    for h, entry in ((torch.zeros(T // 2, 2, H), "sorted"), (torch.zeros(T - 1, 1, H), "rows"),
+                     (torch.zeros(2, T // 2, H), "sorted")):
+        n = h.numel() // H
+        m.experts(h, torch.zeros(n, 1, dtype=torch.int32), torch.zeros(n, 1))
+        assert calls[-1] == entry, h.shape
