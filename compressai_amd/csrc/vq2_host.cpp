@@ -79,6 +79,19 @@ void* stream_of(const at::Device& dev)
     return (void*)py::cast<uintptr_t>(get((int)dev.index()));
 }
 
+// Runs a library call without the interpreter lock, as ctypes does: a launch
+// waits while the GPU's queue is full, and the other Python threads stood
+// still with it (600 ms behind 0.6 s of queued work).  The call may touch no
+// Python object and throws nothing.
+template <class F>
+int unlocked(F call)
+{
+    PyThreadState* const state = PyEval_SaveThread();
+    const int status = call();
+    PyEval_RestoreThread(state);
+    return status;
+}
+
 void check_status(int status, const char* name)
 {
     if (status == VQ2_OK) return;
@@ -151,9 +164,12 @@ py::object sorted_gemv(const at::Tensor& x, const py::sequence& mats, const at::
     const int slices = (int)sorted_slices(chunks, min_ipc, cu);
     const auto ws = sorted_workspace(workspace, *c.dev, vq2_sorted_gemv_workspace(m, (int)k, slices));
     const float sc = rht_scale ? (float)*rht_scale : (hb ? (float)(1.0 / std::sqrt((double)hb)) : 1.0f);
-    check_status(vq2_sorted_gemv(ptr(x), dt_code(x.scalar_type()), (const int32_t*)ptr(perm), (const int8_t*)ptr(sign), hb, sc,
-                                 (int)k, m, ptr(cb0), s2 ? ptr(cb1) : nullptr, dt_code(cb0.scalar_type()), dt_code(s_dt),
-                                 dt_code(out_dtype), n, (float)rs, slices, ws.first, ws.second, stream_of(*c.dev)),
+    void* const st = stream_of(*c.dev);
+    check_status(unlocked([&] {
+                     return vq2_sorted_gemv(ptr(x), dt_code(x.scalar_type()), (const int32_t*)ptr(perm), (const int8_t*)ptr(sign),
+                                            hb, sc, (int)k, m, ptr(cb0), s2 ? ptr(cb1) : nullptr, dt_code(cb0.scalar_type()),
+                                            dt_code(s_dt), dt_code(out_dtype), n, (float)rs, slices, ws.first, ws.second, st);
+                 }),
                  "vq2_sorted_gemv");
     return ys;
 }
@@ -232,10 +248,12 @@ py::object gemv_rht(const at::Tensor& x, const py::sequence& mats, const at::Ten
     py::list ys = make_outputs(r, x, x.dim() == 2 ? std::optional<int64_t>(batch) : std::nullopt, out_dtype);
     if (x.dim() != 2 && batch != 1) return py::none();
     const float sc = rht_scale ? (float)*rht_scale : (float)(1.0 / std::sqrt((double)hb));
-    check_status(vq2_gemv_rht(ptr(x), dt_code(x.scalar_type()), batch, n, (const int32_t*)ptr(perm),
-                              (const int8_t*)ptr(sign), hb, sc, (int)r.k, r.seg, r.s2, ptr(cb0), ptr(cb1),
-                              dt_code(cb0.scalar_type()), dt_code(r.s_dt), dt_code(out_dtype), n, (float)rs,
-                              stream_of(*c.dev)),
+    void* const st = stream_of(*c.dev);
+    check_status(unlocked([&] {
+                     return vq2_gemv_rht(ptr(x), dt_code(x.scalar_type()), batch, n, (const int32_t*)ptr(perm),
+                                         (const int8_t*)ptr(sign), hb, sc, (int)r.k, r.seg, r.s2, ptr(cb0), ptr(cb1),
+                                         dt_code(cb0.scalar_type()), dt_code(r.s_dt), dt_code(out_dtype), n, (float)rs, st);
+                 }),
                  "vq2_gemv_rht");
     return ys;
 }
@@ -262,10 +280,13 @@ py::object rows_gemm(const at::Tensor& x, const py::sequence& mats, const at::Te
     py::list ys = make_outputs(r, x, batch, out_dtype);
     const at::Tensor ws = at::empty({(int64_t)bytes}, x.options().dtype(at::kByte));
     const float sc = rht_scale ? (float)*rht_scale : (hb ? (float)(1.0 / std::sqrt((double)hb)) : 1.0f);
-    check_status(vq2_rows_gemm(ptr(x), dt_code(x.scalar_type()), batch, n, (const int32_t*)ptr(perm),
-                               (const int8_t*)ptr(sign), hb, sc, dt_code(act_dtype), (int)r.k, r.seg, r.s2, ptr(cb0),
-                               ptr(cb1), cdt, dt_code(r.s_dt), dt_code(out_dtype), n, (float)rs, ws.data_ptr(), bytes,
-                               stream_of(*c.dev)),
+    void* const st = stream_of(*c.dev);
+    check_status(unlocked([&] {
+                     return vq2_rows_gemm(ptr(x), dt_code(x.scalar_type()), batch, n, (const int32_t*)ptr(perm),
+                                          (const int8_t*)ptr(sign), hb, sc, dt_code(act_dtype), (int)r.k, r.seg, r.s2,
+                                          ptr(cb0), ptr(cb1), cdt, dt_code(r.s_dt), dt_code(out_dtype), n, (float)rs,
+                                          ws.data_ptr(), bytes, st);
+                 }),
                  "vq2_rows_gemm");
     return ys;
 }
@@ -352,16 +373,20 @@ py::object sorted_moe(const at::Tensor& h, py::handle gate_up, const at::Tensor&
     const int sg = py::cast<int>(sl[0]), sd = py::cast<int>(sl[1]);
     const auto ws = sorted_workspace(workspace, *c.dev, vq2_sorted_moe_workspace(T, (int)P, H, I, sg, sd));
     at::Tensor out = at::empty({T, H}, h.options().dtype(out_dtype));
-    check_status(
-        vq2_sorted_moe(ptr(h), dt_code(h.scalar_type()), T, (int)P, router ? nullptr : ptr(ids),
-                       !router && ids->scalar_type() == at::kLong, router ? nullptr : (const float*)ptr(w),
-                       router ? ptr(logits) : nullptr, router ? dt_code(logits->scalar_type()) : 0, n_routed,
-                       router ? (int)*top_k : 0, router ? *shared_id : 0, router ? ptr(gate) : nullptr,
-                       router ? dt_code(gate->scalar_type()) : 0, router ? ids_out.data_ptr<int32_t>() : nullptr,
-                       router ? w_out.data_ptr<float>() : nullptr, gp.experts, H, I, &gp.p, &dp.p, ptr(cb),
-                       dt_code(cb.scalar_type()), &rh, &ri, out.data_ptr(), dt_code(out_dtype), sg, sd, ws.first, ws.second,
-                       stream_of(*c.dev)),
-        "vq2_sorted_moe");
+    int32_t* const io = router ? ids_out.data_ptr<int32_t>() : nullptr;
+    float* const wo = router ? w_out.data_ptr<float>() : nullptr;
+    void* const st = stream_of(*c.dev);
+    check_status(unlocked([&] {
+                     return vq2_sorted_moe(
+                         ptr(h), dt_code(h.scalar_type()), T, (int)P, router ? nullptr : ptr(ids),
+                         !router && ids->scalar_type() == at::kLong, router ? nullptr : (const float*)ptr(w),
+                         router ? ptr(logits) : nullptr, router ? dt_code(logits->scalar_type()) : 0, n_routed,
+                         router ? (int)*top_k : 0, router ? *shared_id : 0, router ? ptr(gate) : nullptr,
+                         router ? dt_code(gate->scalar_type()) : 0, io, wo, gp.experts, H, I, &gp.p, &dp.p, ptr(cb),
+                         dt_code(cb.scalar_type()), &rh, &ri, out.data_ptr(), dt_code(out_dtype), sg, sd, ws.first, ws.second,
+                         st);
+                 }),
+                 "vq2_sorted_moe");
     if (router) return py::make_tuple(out, ids_out, w_out);
     return py::cast(out);
 }

@@ -3,6 +3,9 @@ the Python entries they stand in for: the same launch, so bit-identical results
 (given outputs take the Python entry), over types, strides of the batch and
 one to four matrices; calls they decline raise what the Python entry raises;
 each stream has its own workspace."""
+import threading
+import time
+
 import pytest
 import torch
 
@@ -78,6 +81,45 @@ def test_sorted_moe(dev, T):
     kw = dict(logits=lg, top_k=2, shared_id=E - 1, shared_gate=synth.activations(8859, 2048).to(dev))
     ref = K.vq_sorted_moe(*args, out=torch.empty(T, 2048, device=dev), **kw)
     assert all(torch.equal(a, b) for a, b in zip(K.vq_sorted_moe(*args, **kw), ref))
+
+
+def test_other_threads_run_while_a_launch_waits(dev):
+    """A launch waits while the GPU's queue is full; other Python threads go
+    on meanwhile, as they do behind the Python entry's launch (the longest
+    pause of a ticking thread against the longest launch: 605 of 600 ms with
+    the interpreter lock held, 1 without)."""
+    n, rows = 2048, 64
+    ms, cb0, _ = _mats(dev, 8860, n, (rows,), 2)
+    mats = [(ms[0]["idx0"].to(dev), None, ms[0]["scale"].to(dev), rows)]
+    x = torch.zeros(1, n, dtype=torch.float16, device=dev)
+    a = torch.zeros(8192, 8192, dtype=torch.bfloat16, device=dev)
+    K.vq_gemv_rht(x, mats, cb0, None, n)
+    torch.cuda.synchronize(dev)
+    pause, stop = [0.0], threading.Event()
+
+    def tick():
+        last = time.perf_counter()
+        while not stop.is_set():
+            time.sleep(0.001)
+            now = time.perf_counter()
+            pause[0] = max(pause[0], now - last)
+            last = now
+
+    t = threading.Thread(target=tick)
+    t.start()
+    try:
+        for _ in range(800):  # ~0.6 s of work, then more launches than the queue holds
+            torch.mm(a, a)
+        longest = 0.0
+        for _ in range(20000):
+            t0 = time.perf_counter()
+            K.vq_gemv_rht(x, mats, cb0, None, n)
+            longest = max(longest, time.perf_counter() - t0)
+    finally:
+        stop.set()
+        t.join()
+    torch.cuda.synchronize(dev)
+    assert pause[0] < max(0.1, longest / 4), (pause[0], longest)
 
 
 def test_declined_calls(dev):
