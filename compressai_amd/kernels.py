@@ -54,7 +54,7 @@ __all__ = [
 
 def _library_available() -> bool:
     try:
-        _lib.load()
+        _lib.host()  # the library, and the native entries of the small calls
         return True
     except (ImportError, OSError):
         return False

@@ -174,6 +174,20 @@ def test_packed_linear_holds_bf16_scales():
     assert keep.scale.dtype == torch.float16 and torch.equal(keep.scale, m["scale"])
 
 
+def test_library_counts_as_available_only_with_the_native_host_module(monkeypatch):
+    """HAVE_TRITON, "fused GPU kernels available": without _vq2_host the
+    entries of the small calls raise ImportError, so it is False."""
+    from compressai_amd import _lib, kernels as K
+
+    assert K._library_available()
+
+    def missing():
+        raise ImportError("no module named _vq2_host")
+
+    monkeypatch.setattr(_lib, "host", missing)
+    assert not K._library_available()
+
+
 def test_packed_linear_release_planes_needs_a_sorted_copy():
     """release_planes() keeps the planes of a module without a code-sorted
     copy (here: on the CPU, where none is built) and says why."""
