@@ -107,7 +107,8 @@ std::pair<void*, size_t> sorted_workspace(py::handle get, const at::Device& dev,
     return {t.data_ptr(), (size_t)t.numel()};
 }
 
-// kernels.sorted_slices
+// The rule of kernels.sorted_slices (tests/test_launch_chunks.py compares the
+// two); chunks >= 1.
 int64_t sorted_slices(int64_t chunks, int64_t min_ipc, int64_t cu)
 {
     const int64_t fit = cu / chunks;
@@ -399,4 +400,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("gemv_rht", &gemv_rht);
     m.def("rows_gemm", &rows_gemm);
     m.def("sorted_moe", &sorted_moe);
+    m.def("sorted_slices", [](int64_t chunks, int64_t min_ipc, int64_t cu) {
+        return sorted_slices(std::max<int64_t>(1, chunks), min_ipc, cu);
+    });
 }

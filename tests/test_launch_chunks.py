@@ -37,6 +37,21 @@ def test_sorted_slices_rule(monkeypatch):
     assert K.sorted_slices([P(n_chunks=512, iters_per_chunk=300)], dev) == 1      # LM head
 
 
+def test_native_slice_rule_is_the_same(monkeypatch):
+    """The native entry chooses its slices itself: the same count for every launch."""
+    from types import SimpleNamespace as P
+
+    from compressai_amd import _lib
+
+    dev = torch.device("cuda", 0)
+    for cu in (1, 32, 256, 304):
+        monkeypatch.setitem(K._CU_COUNT, 0, cu)
+        for chunks in [*range(1, 130), 256, 257, 600]:
+            for ipc in (1, 19, 20, 39, 40, 59, 60, 171, 640, 700):
+                planes = [P(n_chunks=chunks, iters_per_chunk=ipc)]
+                assert _lib.host().sorted_slices(chunks, ipc, cu) == K.sorted_slices(planes, dev), (cu, chunks, ipc)
+
+
 def test_sorted_batch_fits_rule():
     """The batch kernel's LDS rule as the runtime reads it: 4-row workgroups above 80 KiB run as
     2-row launches, which must fit in 150 KiB."""
