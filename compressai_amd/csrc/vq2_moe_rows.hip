@@ -428,7 +428,9 @@ __global__ void __launch_bounds__(MR_THREADS, MT == 2 ? 4 : 2) moe_gemm_kernel(c
             const int r = i * 16 + q * 4 + e;
             if (r >= tile.count) continue;
             const int slot = tile.slot0 + r;
-            float v = acc[i][e] + err[i][e];
+            // (an infinite sum stays one: its two-sum error is NaN)
+            float v = acc[i][e];
+            if (fabsf(v) < __builtin_inff()) v += err[i][e];
             if constexpr (F16) v = ldexpf(v, -a.e[a.row_of ? a.row_of[slot] : slot]);
             v *= s;
             if (a.w) v *= a.w[a.slot_pair[slot]];

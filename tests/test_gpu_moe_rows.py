@@ -154,3 +154,25 @@ def test_layer_with_a_top_k_above_the_router_entrys_runs_for_any_token_count(dev
     out = layer(h, lg)
     few = torch.cat([layer(h[t:t + 4], lg[t:t + 4]) for t in range(0, T, 4)])
     assert float((out - few).abs().max()) <= TOL * float(few.abs().max())
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_a_product_past_fp32_is_infinite_as_in_the_one_pair_kernels(dev, sign):
+    """Every centroid value 1e15 (bf16 codebooks reach that far): the gate_up
+    sums are 1e13, their activation rotates to one value of ~8e26 and zeros,
+    and the down product leaves fp32.  The result is infinite, not NaN."""
+    E, H, I, P = 3, 64, 64, 2
+    T = 20
+    gu, dn = synth.indices16(9901, (E, 2 * I, H // 8)), synth.indices16(9902, (E, H, I // 8))
+    gus, dns = torch.full((E, 2 * I), 1e-2 / 8), torch.ones(E, H)
+    cb = torch.full((65536, 8), 1e15, dtype=torch.bfloat16)
+    mod = ResidentMoEExperts.from_pools(gu.to(dev), gus.to(dev), dn.to(dev), dns.to(dev), cb.to(dev), sorted_layout=True)
+    rot = (None, None, 64, 0.125)
+    h = torch.ones(T, H, device=dev)
+    ids = torch.randint(0, E, (T, P), generator=synth.gen(9903)).to(dev)
+    w = torch.full((T, P), 0.5 * sign, device=dev)
+    one = K.vq_sorted_moe(h, mod.sorted_gu, mod.gate_up_scale, mod.sorted_dn, mod.down_scale, mod.cb16, rot, rot,
+                          ids=ids, w=w)
+    assert bool((one == sign * float("inf")).all())
+    out = K.vq_moe_rows(h, ids, w, mod.gate_up_idx, mod.gate_up_scale, mod.down_idx, mod.down_scale, mod.cb16, rot, rot)
+    assert torch.equal(out, one)
