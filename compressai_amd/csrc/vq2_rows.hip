@@ -199,7 +199,7 @@ struct RowsArgs {
     int kw;  // waves of a workgroup that share a column tile's k tiles
     int nc;  // column tiles of a workgroup of rows_gemm_kernel
     int nz;  // workgroups that share a tile's k tiles (gridDim.z); nc is 1 then
-    float* part;    // nz > 1: [row block][column tile][nz][16 MT][16 NT] sums
+    float* part;    // nz > 1: [row block][column tile][nz][16 MT][16] sums
     uint32_t* cnt;  // nz > 1: arrivals per [row block][column tile], zero
     int tiles;      // column tiles of all matrices
     RowsSeg seg[4];
@@ -241,13 +241,13 @@ constexpr int RW_MAX_MT = 4;     // 16-row tiles of a wave of rows_gemm_kernel
 constexpr int RW_WIDE_WAVES = 4; // waves of a rows_wide_kernel workgroup
 constexpr int RW_MAX_Z = 4;  // workgroups that share a tile's k tiles
 
-// Up to 16 * MT rows: a workgroup is nc column tiles of 16 * NT columns x kw
-// waves over the k tiles; blockIdx.y counts blocks of 16 * MT rows.
-template <int S2, int MT, int NT>
+// Up to 16 * MT rows: a workgroup is nc column tiles of 16 columns x kw waves
+// over the k tiles; blockIdx.y counts blocks of 16 * MT rows.
+template <int S2, int MT>
 __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const RowsArgs a)
 {
     touch_kernargs(a);
-    extern __shared__ __align__(16) float s_red[];  // [waves][16 MT][16 NT + 1]
+    extern __shared__ __align__(16) float s_red[];  // [waves][16 MT][17]
     __shared__ half8_t s_c1[S2 == VQ2_S2_U8 ? 256 : 1];
     __shared__ int s_e[16 * MT];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -257,7 +257,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     const int tile = (int)blockIdx.x * nc + ct0;
     const int k0 = (int)blockIdx.z * kw + wave - ct0 * kw, kstep = kw * a.nz;
     const RowsSeg& sg = rows_seg(a, tile);
-    const int col0 = (tile - sg.tile0) * 16 * NT;  // may lie past the last matrix's rows (tail workgroup)
+    const int col0 = (tile - sg.tile0) * 16;  // may lie past the last matrix's rows (tail workgroup)
     const int mt0 = (int)blockIdx.y * MT;
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
 
@@ -266,33 +266,25 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     // Finding the matrix of each output again, with its divisions and its
     // loads, took 4.4 of 35.9 us for gate and up of 6144 x 2048 at 3 bpw and 64 rows.
     const int e_pre = tid < 16 * MT ? a.e[min(mt0 * 16 + tid, a.m - 1)] : 0;
-    const int ecol = min(col0 + tid % (16 * NT), sg.rows - 1);
+    const int ecol = min(col0 + tid % 16, sg.rows - 1);
     const uint32_t s_pre = nc == 1 ? load_raw(sg.scale, a.s_dt, ecol) : 0u;
 
-    int64_t rowoff[NT];
-#pragma unroll
-    for (int c = 0; c < NT; c++) {
-        const int r = col0 + c * 16 + nl;
-        rowoff[c] = (int64_t)(r < sg.rows ? r : 0) * a.ng;
-    }
+    const int64_t rowoff = (int64_t)(col0 + nl < sg.rows ? col0 + nl : 0) * a.ng;
     // row tiles past the last one read tile mt_last again (results dropped)
     const int mt_last = (a.m - 1) >> 4;
     const half8_t* ap[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) ap[i] = a.a + (int64_t)min(mt0 + i, mt_last) * a.kt * 512 + lane;
 
-    f32x4_t acc[MT][NT];
+    f32x4_t acc[MT];
 #pragma unroll
-    for (int i = 0; i < MT; i++)
-#pragma unroll
-        for (int c = 0; c < NT; c++) acc[i][c] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i = 0; i < MT; i++) acc[i] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 
-    RowCodes<S2> cd[NT];
+    RowCodes<S2> cd;
     auto load_codes = [&](int kt) {
         // the last k tile may be short: whole k blocks of 8 groups are missing
         const int g = kt * RW_TILE_G + q * 8;
-#pragma unroll
-        for (int c = 0; c < NT; c++) cd[c].load(sg, rowoff[c] + (g < a.ng ? g : 0));
+        cd.load(sg, rowoff + (g < a.ng ? g : 0));
     };
     if (k0 < a.kt) load_codes(k0);
     if constexpr (S2 == VQ2_S2_U8) {
@@ -301,47 +293,38 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     }
     for (int kt = k0; kt < a.kt; kt += kstep) {
         const bool g_ok = kt * RW_TILE_G + q * 8 < a.ng;
-        half8_t b0[8][NT], b1[8][NT];
+        half8_t b0[8], b1[8];
 #pragma unroll
-        for (int t = 0; t < 8; t++)
-#pragma unroll
-            for (int c = 0; c < NT; c++) {
-                b0[t][c] = a.cb0[cd[c].c0(t)];
-                if constexpr (S2 == VQ2_S2_U16) b1[t][c] = a.cb1[cd[c].c1(t)];
-                if constexpr (S2 == VQ2_S2_U8) b1[t][c] = s_c1[cd[c].c1(t)];
-            }
+        for (int t = 0; t < 8; t++) {
+            b0[t] = a.cb0[cd.c0(t)];
+            if constexpr (S2 == VQ2_S2_U16) b1[t] = a.cb1[cd.c1(t)];
+            if constexpr (S2 == VQ2_S2_U8) b1[t] = s_c1[cd.c1(t)];
+        }
         if (kt + kstep < a.kt) load_codes(kt + kstep);
 #pragma unroll
         for (int t = 0; t < 8; t++) {
             half8_t av[MT];
 #pragma unroll
             for (int i = 0; i < MT; i++) av[i] = ap[i][((int64_t)kt * 8 + t) * 64];
+            const half8_t bb = g_ok ? b0[t] : zero8;
 #pragma unroll
-            for (int c = 0; c < NT; c++) {
-                const half8_t bb = g_ok ? b0[t][c] : zero8;
+            for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bb, acc[i], 0, 0, 0);
+            if constexpr (S2 != VQ2_S2_NONE) {
+                const half8_t bc = g_ok ? b1[t] : zero8;
 #pragma unroll
-                for (int i = 0; i < MT; i++)
-                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bb, acc[i][c], 0, 0, 0);
-                if constexpr (S2 != VQ2_S2_NONE) {
-                    const half8_t bc = g_ok ? b1[t][c] : zero8;
-#pragma unroll
-                    for (int i = 0; i < MT; i++)
-                        acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bc, acc[i][c], 0, 0, 0);
-                }
+                for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bc, acc[i], 0, 0, 0);
             }
         }
     }
 
     // D[i][j]: activation row 4 (l / 16) + e of the tile, column l % 16; the
     // waves' sums meet in LDS and are added in wave order
-    constexpr int LD = 16 * NT + 1, TILE = 16 * MT * LD;
+    constexpr int LD = 17, TILE = 16 * MT * LD;
     float* mine = s_red + wave * TILE;
 #pragma unroll
     for (int i = 0; i < MT; i++)
 #pragma unroll
-        for (int c = 0; c < NT; c++)
-#pragma unroll
-            for (int e = 0; e < 4; e++) mine[(i * 16 + q * 4 + e) * LD + c * 16 + nl] = acc[i][c][e];
+        for (int e = 0; e < 4; e++) mine[(i * 16 + q * 4 + e) * LD + nl] = acc[i][e];
     if (tid < 16 * MT) s_e[tid] = e_pre;
     __syncthreads();
     const int mrows = min(16 * MT, a.m - mt0 * 16);
@@ -351,33 +334,33 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         // this workgroup's sums; the last of the tile's workgroups adds them
         // in order (arrive_last)
         const int64_t unit = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
-        float* pt = a.part + (unit * a.nz + blockIdx.z) * (256 * MT * NT);
-        for (int t = tid; t < 256 * MT * NT; t += (int)blockDim.x) {
-            const float* p = s_red + t / (16 * NT) * LD + t % (16 * NT);
+        float* pt = a.part + (unit * a.nz + blockIdx.z) * (256 * MT);
+        for (int t = tid; t < 256 * MT; t += (int)blockDim.x) {
+            const float* p = s_red + t / 16 * LD + t % 16;
             float sum = 0.0f;
             for (int w = 0; w < kw; w++) sum += p[w * TILE];
             share_store(pt + t, sum);
         }
         if (!arrive_last(a.cnt + unit, (uint32_t)a.nz)) return;
-        pt = a.part + unit * a.nz * (256 * MT * NT);
-        for (int t = tid; t < 256 * MT * NT; t += (int)blockDim.x) {
+        pt = a.part + unit * a.nz * (256 * MT);
+        for (int t = tid; t < 256 * MT; t += (int)blockDim.x) {
             // at most RW_MAX_Z partials, their loads in flight together
             float v[RW_MAX_Z], sum = 0.0f;
 #pragma unroll
-            for (int z = 0; z < RW_MAX_Z; z++) v[z] = share_load(pt + min(z, a.nz - 1) * (256 * MT * NT) + t);
+            for (int z = 0; z < RW_MAX_Z; z++) v[z] = share_load(pt + min(z, a.nz - 1) * (256 * MT) + t);
 #pragma unroll
             for (int z = 0; z < RW_MAX_Z; z++) sum += z < a.nz ? v[z] : 0.0f;
-            s_red[t / (16 * NT) * LD + t % (16 * NT)] = sum;
+            s_red[t / 16 * LD + t % 16] = sum;
         }
         __syncthreads();
         nred = 1;
     }
     if (nc == 1) {
-        // (blockDim is a multiple of 16 NT: the thread's column stays)
-        const int c = tid % (16 * NT);
+        // (blockDim is a multiple of 16: the thread's column stays)
+        const int c = tid % 16;
         const float s = raw_as_f32(s_pre, a.s_dt);
         if (col0 + c >= sg.rows) return;
-        for (int r = tid / (16 * NT); r < mrows; r += (int)blockDim.x / (16 * NT)) {
+        for (int r = tid / 16; r < mrows; r += (int)blockDim.x / 16) {
             const float* p = red + r * LD + c;
             float sum = 0.0f;
             for (int w = 0; w < nred; w++) sum += p[w * TILE];
@@ -385,12 +368,12 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         }
         return;
     }
-    for (int t = tid; t < nc * mrows * 16 * NT; t += (int)blockDim.x) {
-        const int c = t % (16 * NT), u = t / (16 * NT);
+    for (int t = tid; t < nc * mrows * 16; t += (int)blockDim.x) {
+        const int c = t % 16, u = t / 16;
         const int r = u % mrows, ct = u / mrows;
         const int tl = (int)blockIdx.x * nc + ct;
         const RowsSeg& so = rows_seg(a, tl);
-        const int col = (tl - so.tile0) * 16 * NT + c;
+        const int col = (tl - so.tile0) * 16 + c;
         if (col >= so.rows) continue;
         const float* p = red + ct * kw * TILE + r * LD + c;
         float sum = 0.0f;
@@ -577,7 +560,7 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(const RowsArgs a)
 // ------------------------------------------------------------------ launch
 struct RowsPlan {
     int kt;
-    int mt, nt;        // 16-row and 16-column tiles of a wave
+    int mt;            // 16-row tiles of a wave
     int kw, nc, nz;    // waves and workgroups over a column tile's k tiles; column tiles of a workgroup
     int wide;          // rows_wide_kernel
     int64_t tiles;     // column tiles of all matrices
@@ -636,8 +619,7 @@ static RowsPlan rows_plan(const RowsCall& c)
     // row blocks of at most 64 rows, as even as whole tiles allow
     const int64_t mtiles = (c.m + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
     p.mt = (int)((mtiles + blocks - 1) / blocks);
-    p.nt = 1;
-    for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 16 * p.nt - 1) / (16 * p.nt);
+    for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 15) / 16;
     p.grid_y = (c.m + 16 * p.mt - 1) / (16 * p.mt);
     // Few column tiles leave CUs idle, and a CU gathers at most ~0.9 codes a
     // ns however few others do: several workgroups then share a tile's k
@@ -646,7 +628,7 @@ static RowsPlan rows_plan(const RowsCall& c)
     // 4096 gathers 13.7 us a call, two workgroups 14.4; at 4 bpw 18.3 / 17.5;
     // 2048 x 6144 at 4 bpw 34.5 / 28.3; 512 x 6144 40.1 / 26.3 / 20.7 with
     // four) and the launch stays within a workgroup per CU.
-    const int64_t gathers = 16 * p.nt * (c.n / 8) * (c.s2 == VQ2_S2_U16 ? 2 : 1);
+    const int64_t gathers = 16 * (c.n / 8) * (c.s2 == VQ2_S2_U16 ? 2 : 1);
     p.nz = 1;
     while (2 * p.nz <= std::min(RW_MAX_Z, p.kt) && 2 * p.nz * p.tiles * p.grid_y <= device_cu_count() &&
            gathers / p.nz >= 6144)
@@ -667,7 +649,7 @@ static RowsPlan rows_plan(const RowsCall& c)
     p.h0 = p.a + (size_t)((c.m + 15) / 16) * p.kt * 512 * sizeof(half8_t);
     p.h1 = p.h0 + (cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
     p.part = p.h1 + (!cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
-    p.total = p.part + (p.wide && p.nz > 1 ? (size_t)p.nz * c.m * p.tiles * 16 : (size_t)units * p.nz * 256 * p.mt * p.nt) *
+    p.total = p.part + (p.wide && p.nz > 1 ? (size_t)p.nz * c.m * p.tiles * 16 : (size_t)units * p.nz * 256 * p.mt) *
                            sizeof(float);
     return p;
 }
@@ -690,20 +672,20 @@ size_t rows_workspace_bytes(const RowsCall& c)
     return rows_check(c) == VQ2_OK ? rows_plan(c).total : 0;
 }
 
-template <int S2, int MT, int NT>
+template <int S2, int MT>
 static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
     // opt in to more than 64 KiB of dynamic LDS, once per instantiation
     static std::once_flag once;
     static hipError_t attr = hipSuccess;
-    constexpr size_t SHM_WAVE = 16 * MT * (16 * NT + 1) * sizeof(float);
+    constexpr size_t SHM_WAVE = 16 * MT * 17 * sizeof(float);
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT, NT>,
+        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RW_MAX_WAVES * SHM_WAVE));
     });
     if (attr != hipSuccess) return attr;
     const size_t shm = waves * SHM_WAVE;
-    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT, NT>), grid, dim3(64 * waves), shm, st, a);
+    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT>), grid, dim3(64 * waves), shm, st, a);
     return hipGetLastError();
 }
 
@@ -711,10 +693,10 @@ template <int S2>
 static hipError_t rows_launch_s(int mt, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
     switch (mt) {
-    case 1: return rows_launch_t<S2, 1, 1>(a, grid, waves, st);
-    case 2: return rows_launch_t<S2, 2, 1>(a, grid, waves, st);
-    case 3: return rows_launch_t<S2, 3, 1>(a, grid, waves, st);
-    default: return rows_launch_t<S2, 4, 1>(a, grid, waves, st);
+    case 1: return rows_launch_t<S2, 1>(a, grid, waves, st);
+    case 2: return rows_launch_t<S2, 2>(a, grid, waves, st);
+    case 3: return rows_launch_t<S2, 3>(a, grid, waves, st);
+    default: return rows_launch_t<S2, 4>(a, grid, waves, st);
     }
 }
 
@@ -824,7 +806,7 @@ int rows_launch(const RowsCall& c)
         const RowsSegCall& g = c.seg[s];
         if (g.rows == 0) continue;
         a.seg[a.nseg++] = RowsSeg{g.idx0, g.idx1, g.scale, g.y, g.y_stride, (int)g.rows, (int)tile};
-        tile += (g.rows + 16 * p.nt - 1) / (16 * p.nt);
+        tile += (g.rows + 15) / 16;
     }
     a.tiles = (int)p.tiles;
     const dim3 grid((unsigned)p.grid_x, (unsigned)p.grid_y, (unsigned)p.nz);
