@@ -46,8 +46,6 @@
 
 namespace vq2 {
 
-typedef __bf16 bhalf8_t __attribute__((ext_vector_type(8)));
-
 constexpr int MR_TILE_G = 32;   // groups per k tile, as in vq2_rows.hip
 constexpr int MR_NS = 3;        // addends of an activation value
 constexpr int MR_TS = 4;        // steps of a stage
@@ -290,17 +288,6 @@ struct MoeGemmArgs {
     const int* slot_pair;
     float* y;            // [slots][rows]
 };
-
-template <int F16>
-__device__ __forceinline__ f32x4_t mfma_16(u32x4 x, u32x4 b, f32x4_t acc)
-{
-    if constexpr (F16)
-        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x), __builtin_bit_cast(half8_t, b), acc,
-                                                      0, 0, 0);
-    else
-        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bhalf8_t, x),
-                                                       __builtin_bit_cast(bhalf8_t, b), acc, 0, 0, 0);
-}
 
 // Workgroup: one tile of up to 16 MT pairs x 128 rows of its expert, a wave 16
 // rows.  Per stage (MR_TS steps of a k tile) the waves gather their own

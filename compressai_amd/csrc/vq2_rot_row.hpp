@@ -1,5 +1,6 @@
 // vq2_rot_row.hpp -- one workgroup rotates one row: the prologue of the kernels
-// that pack activations for the matrix cores (vq2_rows.hip, vq2_moe_rows.hip).
+// that pack activations for the matrix cores (vq2_rows.hip, vq2_moe_rows.hip),
+// and the matrix instruction they pack for.
 //
 // Thread t holds the 8 values of group t: value bits 0-2 are in its
 // registers, bits 3-8 across the lanes of its wave, 9-10 and 11-12 across
@@ -15,6 +16,19 @@
 namespace vq2 {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
+typedef __bf16 bhalf8_t __attribute__((ext_vector_type(8)));
+
+// v_mfma_f32_16x16x32 of 16-byte operands, fp16 (F16) or bf16
+template <int F16>
+__device__ __forceinline__ f32x4_t mfma_16(u32x4 x, u32x4 b, f32x4_t acc)
+{
+    if constexpr (F16)
+        return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, x), __builtin_bit_cast(half8_t, b), acc,
+                                                      0, 0, 0);
+    else
+        return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bhalf8_t, x),
+                                                       __builtin_bit_cast(bhalf8_t, b), acc, 0, 0, 0);
+}
 
 constexpr int ROT_ROW_MAX_T = 1024;  // threads, and groups of the widest row
 

@@ -8,7 +8,10 @@
 //  1. rows_pack_kernel: one workgroup per activation row rotates it (or takes
 //     it rotated), finds the row's power-of-two scale and writes it as fp16
 //     in the order the second launch's matrix instructions read (below).
-//     Codebooks that are not fp16 are rounded to fp16 by further workgroups
+//     Up to RW_BF_ROWS rows a bf16 codebook is multiplied as it is, in bf16:
+//     each fp16 value of a row goes in as two bf16 addends, which hold its 11
+//     bits exactly, in two packed rows whose sums the product adds.  Else
+//     codebooks that are not fp16 are rounded to fp16 by further workgroups
 //     of the same launch, so the second launch gathers 16 bytes a code.
 //  2. rows_gemm_kernel, or for many rows rows_wide_kernel (and rows_sum_kernel
 //     where its k tiles are shared): the product.
@@ -41,7 +44,9 @@
 //
 // Precision: as vq2_gemm_mfma.hip: the rotation in fp32, one rounding to fp16
 // under a power-of-two scale per row (divided out of the fp32 sum exactly),
-// fp16 centroids as they are, fp32 accumulation.
+// fp16 centroids as they are, fp32 accumulation.  Up to RW_BF_ROWS rows bf16
+// centroids as they are too, as in the sorted batch kernel; above, rounded to
+// fp16 as in vq2_gemm_mfma.hip.
 //
 // Semantics: the PackedLinear fallback for batch > 1, rotate, dequantize,
 // F.linear (vq2/runtime.py:82-89, 105-110), for (16,), (16,8) and (16,16).
@@ -58,6 +63,15 @@ constexpr int RW_TILE_G = 32;      // groups per k tile
 constexpr int RW_PACK_MAX = ROT_ROW_MAX_T;
 constexpr int64_t RW_MAX_N = 8 * RW_PACK_MAX;
 constexpr int RW_CB_ROWS = 65536;
+// bf16 codebooks: up to this many rows are packed as two bf16 addends each,
+// which fit one 16-row tile, so the centroids need no rounding: exact, and
+// without the pass over the codebooks in every call.  Graph replays, us a
+// call, 8 rows, rounded / two addends (vq2_rht and vq2_gemm_small_m): 6144 x
+// 2048 at 4 bpw 25.5 / 23.3 (25.2), 2048 x 6144 27.5 / 26.1 (26.2), 2048 x
+// 2048 at 2 bpw 12.9 / 11.7 (13.6).  A second tile for 9 to 16 rows gains
+// less than it costs: 6144 x 2048 at 3 bpw, 16 rows 17.8 / 18.3.
+constexpr int64_t RW_BF_ROWS = 8;
+static_assert(2 * RW_BF_ROWS <= 16, "both addends of every row in one row tile");
 
 // ------------------------------------------------------------- the packing
 struct RowsPackArgs {
@@ -74,6 +88,7 @@ struct RowsPackArgs {
     float scale;
     int act_dt;  // type the rotated activation is rounded to first
     half8_t* a;  // packed activation
+    int bf;      // two bf16 addends a value, the second in row m + row
     int* e;      // exponent of each row's scale
     uint32_t* cnt;  // arrival counters of the product, to be cleared
     int n_cnt;
@@ -170,7 +185,24 @@ __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackAr
     half8_t h;
 #pragma unroll
     for (int k = 0; k < 8; k++) h[k] = (_Float16)ldexpf(v[k], e);
-    a.a[(((row >> 4) * a.kt + kt) * 8 + t) * 64 + q * 16 + (row & 15)] = h;
+    auto put = [&](int64_t r, half8_t w) { a.a[(((r >> 4) * a.kt + kt) * 8 + t) * 64 + q * 16 + (r & 15)] = w; };
+    if (!a.bf) return put(row, h);
+    u32x4 hi, lo;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        const float f = (float)h[k];
+        const uint32_t b = f32_to_bf16_bits(f);
+        const uint32_t c = fabsf(f) < __builtin_inff() ? f32_to_bf16_bits(f - bf16_bits_to_f32(b)) : 0u;
+        if (k & 1) {
+            hi[k >> 1] |= b << 16;
+            lo[k >> 1] |= c << 16;
+        } else {
+            hi[k >> 1] = b;
+            lo[k >> 1] = c;
+        }
+    }
+    put(row, __builtin_bit_cast(half8_t, hi));
+    put(a.m + row, __builtin_bit_cast(half8_t, lo));
 }
 
 // ------------------------------------------------------------- the product
@@ -188,9 +220,10 @@ struct RowsArgs {
     const half8_t* a;  // packed activation
     const int* e;
     int m;
+    int mp;  // packed rows: m, with two bf16 addends 2 m
     int kt;  // k tiles
     int ng;
-    const half8_t* cb0;  // fp16 codebooks
+    const half8_t* cb0;  // fp16 codebooks (rows_gemm_kernel<S2, MT, 1>: bf16)
     const half8_t* cb1;
     int s_dt;
     int y_dt;
@@ -242,8 +275,10 @@ constexpr int RW_WIDE_WAVES = 4; // waves of a rows_wide_kernel workgroup
 constexpr int RW_MAX_Z = 4;  // workgroups that share a tile's k tiles
 
 // Up to 16 * MT rows: a workgroup is nc column tiles of 16 columns x kw waves
-// over the k tiles; blockIdx.y counts blocks of 16 * MT rows.
-template <int S2, int MT>
+// over the k tiles; blockIdx.y counts blocks of 16 * MT rows.  BF: bf16
+// codebooks and packed rows, the addends of row r in rows r and m + r of the
+// one row block.
+template <int S2, int MT, int BF>
 __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const RowsArgs a)
 {
     touch_kernargs(a);
@@ -260,6 +295,9 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     const int col0 = (tile - sg.tile0) * 16;  // may lie past the last matrix's rows (tail workgroup)
     const int mt0 = (int)blockIdx.y * MT;
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    auto mfma = [](half8_t x, half8_t b, f32x4_t c) {
+        return mfma_16<!BF>(__builtin_bit_cast(u32x4, x), __builtin_bit_cast(u32x4, b), c);
+    };
 
     // what the epilogue needs, loaded ahead of everything else: the rows'
     // exponents and (one column tile: a thread keeps its column) the scale.
@@ -271,7 +309,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
 
     const int64_t rowoff = (int64_t)(col0 + nl < sg.rows ? col0 + nl : 0) * a.ng;
     // row tiles past the last one read tile mt_last again (results dropped)
-    const int mt_last = (a.m - 1) >> 4;
+    const int mt_last = (a.mp - 1) >> 4;
     const half8_t* ap[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) ap[i] = a.a + (int64_t)min(mt0 + i, mt_last) * a.kt * 512 + lane;
@@ -308,11 +346,11 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
             for (int i = 0; i < MT; i++) av[i] = ap[i][((int64_t)kt * 8 + t) * 64];
             const half8_t bb = g_ok ? b0[t] : zero8;
 #pragma unroll
-            for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bb, acc[i], 0, 0, 0);
+            for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bb, acc[i]);
             if constexpr (S2 != VQ2_S2_NONE) {
                 const half8_t bc = g_ok ? b1[t] : zero8;
 #pragma unroll
-                for (int i = 0; i < MT; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[i], bc, acc[i], 0, 0, 0);
+                for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bc, acc[i]);
             }
         }
     }
@@ -355,15 +393,22 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         __syncthreads();
         nred = 1;
     }
+    // the sum of the output at p, over the waves that shared its k tiles
+    auto total = [&](const float* p) {
+        float sum = 0.0f;
+        for (int w = 0; w < nred; w++) {
+            sum += p[w * TILE];
+            if constexpr (BF) sum += p[w * TILE + a.m * LD];
+        }
+        return sum;
+    };
     if (nc == 1) {
         // (blockDim is a multiple of 16: the thread's column stays)
         const int c = tid % 16;
         const float s = raw_as_f32(s_pre, a.s_dt);
         if (col0 + c >= sg.rows) return;
         for (int r = tid / 16; r < mrows; r += (int)blockDim.x / 16) {
-            const float* p = red + r * LD + c;
-            float sum = 0.0f;
-            for (int w = 0; w < nred; w++) sum += p[w * TILE];
+            const float sum = total(red + r * LD + c);
             store_from_f32(sg.y, a.y_dt, (int64_t)(mt0 * 16 + r) * sg.y_stride + col0 + c, (ldexpf(sum, -s_e[r]) * s) * a.rs);
         }
         return;
@@ -375,9 +420,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         const RowsSeg& so = rows_seg(a, tl);
         const int col = (tl - so.tile0) * 16 + c;
         if (col >= so.rows) continue;
-        const float* p = red + ct * kw * TILE + r * LD + c;
-        float sum = 0.0f;
-        for (int w = 0; w < nred; w++) sum += p[w * TILE];
+        const float sum = total(red + ct * kw * TILE + r * LD + c);
         const float s = load_as_f32(so.scale, a.s_dt, col);
         store_from_f32(so.y, a.y_dt, (int64_t)(mt0 * 16 + r) * so.y_stride + col, (ldexpf(sum, -s_e[r]) * s) * a.rs);
     }
@@ -559,6 +602,8 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(const RowsArgs a)
 
 // ------------------------------------------------------------------ launch
 struct RowsPlan {
+    int bf;            // bf16 products (RW_BF_ROWS)
+    int64_t mp;        // packed rows
     int kt;
     int mt;            // 16-row tiles of a wave
     int kw, nc, nz;    // waves and workgroups over a column tile's k tiles; column tiles of a workgroup
@@ -616,11 +661,13 @@ static RowsPlan rows_plan(const RowsCall& c)
 {
     RowsPlan p{};
     p.kt = (int)((c.n / 8 + RW_TILE_G - 1) / RW_TILE_G);
+    p.bf = c.cb_dt == VQ2_DT_BF16 && c.m <= RW_BF_ROWS;
+    p.mp = p.bf ? 2 * c.m : c.m;
     // row blocks of at most 64 rows, as even as whole tiles allow
-    const int64_t mtiles = (c.m + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
+    const int64_t mtiles = (p.mp + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
     p.mt = (int)((mtiles + blocks - 1) / blocks);
     for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 15) / 16;
-    p.grid_y = (c.m + 16 * p.mt - 1) / (16 * p.mt);
+    p.grid_y = (p.mp + 16 * p.mt - 1) / (16 * p.mt);
     // Few column tiles leave CUs idle, and a CU gathers at most ~0.9 codes a
     // ns however few others do: several workgroups then share a tile's k
     // tiles, while a workgroup has 6144 gathers or more (below that the
@@ -642,11 +689,11 @@ static RowsPlan rows_plan(const RowsCall& c)
     p.nc = (int)std::max<int64_t>(1, std::min<int64_t>(8 / p.kw, p.tiles * p.grid_y / device_cu_count()));
     if (c.m > 16 * RW_MAX_MT) rows_plan_wide(c, p);
     p.grid_x = (p.tiles + p.nc - 1) / p.nc;
-    const bool cvt = c.cb_dt != VQ2_DT_F16;
+    const bool cvt = c.cb_dt != VQ2_DT_F16 && !p.bf;
     const int64_t units = p.nz > 1 && !p.wide ? p.grid_x * p.grid_y : 0;
     p.e = up256((size_t)units * sizeof(uint32_t));
     p.a = p.e + up256((size_t)c.m * sizeof(int));
-    p.h0 = p.a + (size_t)((c.m + 15) / 16) * p.kt * 512 * sizeof(half8_t);
+    p.h0 = p.a + (size_t)((p.mp + 15) / 16) * p.kt * 512 * sizeof(half8_t);
     p.h1 = p.h0 + (cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
     p.part = p.h1 + (!cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
     p.total = p.part + (p.wide && p.nz > 1 ? (size_t)p.nz * c.m * p.tiles * 16 : (size_t)units * p.nz * 256 * p.mt) *
@@ -672,7 +719,7 @@ size_t rows_workspace_bytes(const RowsCall& c)
     return rows_check(c) == VQ2_OK ? rows_plan(c).total : 0;
 }
 
-template <int S2, int MT>
+template <int S2, int MT, int BF = 0>
 static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
     // opt in to more than 64 KiB of dynamic LDS, once per instantiation
@@ -680,18 +727,19 @@ static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStre
     static hipError_t attr = hipSuccess;
     constexpr size_t SHM_WAVE = 16 * MT * 17 * sizeof(float);
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT>,
+        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT, BF>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RW_MAX_WAVES * SHM_WAVE));
     });
     if (attr != hipSuccess) return attr;
     const size_t shm = waves * SHM_WAVE;
-    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT>), grid, dim3(64 * waves), shm, st, a);
+    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT, BF>), grid, dim3(64 * waves), shm, st, a);
     return hipGetLastError();
 }
 
 template <int S2>
-static hipError_t rows_launch_s(int mt, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
+static hipError_t rows_launch_s(int mt, int bf, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
+    if (bf) return rows_launch_t<S2, 1, 1>(a, grid, waves, st);
     switch (mt) {
     case 1: return rows_launch_t<S2, 1>(a, grid, waves, st);
     case 2: return rows_launch_t<S2, 2>(a, grid, waves, st);
@@ -754,7 +802,7 @@ int rows_launch(const RowsCall& c)
         return set_error(VQ2_ERR_ARG, "vq2_rows_gemm: workspace of %zu bytes (256-byte aligned) needed, got %zu", p.total,
                          c.ws_bytes);
     char* ws = (char*)c.workspace;
-    const bool cvt = c.cb_dt != VQ2_DT_F16;
+    const bool cvt = c.cb_dt != VQ2_DT_F16 && !p.bf;
     hipStream_t st = (hipStream_t)c.stream;
 
     RowsPackArgs k{};
@@ -771,6 +819,7 @@ int rows_launch(const RowsCall& c)
     k.scale = c.xscale;
     k.act_dt = c.act_dt;
     k.a = (half8_t*)(ws + p.a);
+    k.bf = p.bf;
     k.e = (int*)(ws + p.e);
     k.cnt = (uint32_t*)ws;
     k.n_cnt = p.nz > 1 && !p.wide ? (int)(p.grid_x * p.grid_y) : 0;
@@ -789,6 +838,7 @@ int rows_launch(const RowsCall& c)
     a.a = k.a;
     a.e = k.e;
     a.m = (int)c.m;
+    a.mp = (int)p.mp;
     a.ng = (int)(c.n / 8);
     a.kt = p.kt;
     a.cb0 = cvt ? k.h0 : (const half8_t*)c.cb0;
@@ -825,9 +875,9 @@ int rows_launch(const RowsCall& c)
         return VQ2_OK;
     }
     switch (c.s2) {
-    case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, a, grid, p.kw * p.nc, st); break;
-    case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, a, grid, p.kw * p.nc, st); break;
-    default: err = rows_launch_s<VQ2_S2_NONE>(p.mt, a, grid, p.kw * p.nc, st); break;
+    case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
+    case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
+    default: err = rows_launch_s<VQ2_S2_NONE>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
     }
     if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm launch");
     return VQ2_OK;

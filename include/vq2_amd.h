@@ -165,7 +165,8 @@ int vq2_gemv_rht(const void* x, int x_dt, int64_t batch, int64_t x_stride,
  *   xr[b] = RHT_fwd(x[b]) as in vq2_gemv_rht (hb == 0: x is rotated), rounded
  *           to act_dt, then to fp16 under a power-of-two scale per row
  *   segs[s].y[b, r] = (sum_k W_s[r, k] * xr[b, k]) * segs[s].scale[r] * rs
- * Codebooks that are not fp16 are rounded to fp16; sums are fp32.  Two or
+ * Codebooks that are not fp16 are rounded to fp16, bf16 ones from 9 rows on
+ * (exact up to 8); sums are fp32.  Two or
  * three launches: the rotated rows go to the workspace in the order the product's
  * matrix instructions read them.  Requires n % 64 == 0, n <= 8192, hb a power
  * of two from 64 on (or 0), 16-byte aligned index planes; x needs no

@@ -130,6 +130,32 @@ def test_projections_of_many_rows_equal_their_own_calls(dev, cfg, n, outs, M):
         assert float((y - ref).abs().max()) <= TOL_SUM * float(ref.abs().max())
 
 
+@pytest.mark.parametrize("cfg,n,outs", [((16,), 2048, (2048, 512, 500)), ((16, 8), 512, (300, 17)),
+                                        ((16, 16), 6144, (500, 512)), ((16, 16), 128, (33,))])
+@pytest.mark.parametrize("M", [3, 8])
+def test_bf16_centroids_enter_as_they_are(dev, cfg, n, outs, M):
+    """Up to 8 rows, bf16 codebooks whose values fp16 cannot hold (above
+    65504, and below its smallest) count with all their bits, as in the sorted
+    batch kernel, which takes projections of a few rows without planes."""
+    big, tiny = 2.0 ** 30, 2.0 ** -30
+    for scale in (big, tiny):
+        cbs = {"16": (synth.codebook(9940).float() * scale).bfloat16(),
+               "16_8": (synth.codebook(9941, rows=256).float() * scale).bfloat16(),
+               "16_16": (synth.codebook(9942).float() * scale).bfloat16()}
+        on = {k: v.to(dev) for k, v in cbs.items()}
+        bpw = {(16,): 2, (16, 8): 3, (16, 16): 4}[cfg]
+        ms = [synth.vq_matrix(9943 + i, out, n, bpw=bpw) for i, out in enumerate(outs)]
+        lins = [PackedLinear((out, n), cfg, "t", [p for p in (m["idx0"], m["idx1"]) if p is not None], m["scale"], on,
+                             dev) for m, out in zip(ms, outs)]
+        x = synth.activations(9950, (M, n), dtype=torch.float32).to(dev)
+        xr = lins[0].rot.fwd(x).cpu().numpy()
+        cb1 = {2: None, 3: cbs["16_8"], 4: cbs["16_16"]}[bpw]
+        for y, m, lin in zip(PackedProjections(lins)(x), ms, lins):
+            _, ref = O.vq_gemv(fp16_row_scaled(xr), m["idx0"], m["idx1"], cbs["16"], cb1, lin.scale.cpu())
+            err = np.abs(y.cpu().numpy() - ref).max(1)
+            assert np.all(err <= TOL_SUM * np.abs(ref).max(1)), (scale, err.max() / np.abs(ref).max())
+
+
 def test_rows_gemm_capture_replays_and_repeats(dev):
     """A captured call whose tiles are summed over workgroups gives the eager
     result bit for bit on every replay, with new inputs and eager calls
