@@ -10,11 +10,12 @@
 //     in the order the second launch's matrix instructions read (below).
 //     Up to RW_BF_ROWS rows a bf16 codebook is multiplied as it is, in bf16:
 //     each fp16 value of a row goes in as two bf16 addends, which hold its 11
-//     bits exactly, in two packed rows whose sums the product adds.  Else
-//     codebooks that are not fp16 are rounded to fp16 by further workgroups
-//     of the same launch, so the second launch gathers 16 bytes a code.
+//     bits exactly, in two packed rows whose sums the product adds.
 //  2. rows_gemm_kernel, or for many rows rows_wide_kernel (and rows_sum_kernel
-//     where its k tiles are shared): the product.
+//     where its k tiles are shared): the product.  rows_gemm_kernel rounds
+//     codebooks that are not fp16 to fp16 as it gathers them.  For
+//     rows_wide_kernel, and fp32 ones of many gathers (RW_F32_GATHERS),
+//     further workgroups of the first launch round them, once per call.
 //
 // Why two launches and this layout.  The products are bound by the random
 // 16-byte centroid gathers, which the L2s serve at ~240 G/s whatever else the
@@ -28,9 +29,13 @@
 // in LDS), so nothing is written but y.  Measured, us a call, rotation
 // included (before: vq2_rht, vq2_gemm_small_m per 64 rows and its reduce
 // launch): 2048 x 6144 at 4 bpw, 16 rows 34.0 -> 25.7; two 6144 x 2048 at
-// 3 bpw, 64 rows, bf16 75.2 -> 31.5; 2999 x 4096 at 2 bpw, 100 rows 52.0 ->
-// 33.1; two 6144 x 2048 at 4 bpw, 1024 rows 979 -> 174; in graph replays
-// 2048 x 2048 at 2 bpw, 16 rows 15.3 -> 13.5.  Bound by the gathers (13 us
+// 3 bpw, 64 rows, bf16 75.2 -> 30.1; 2999 x 4096 at 2 bpw, 100 rows 52.0 ->
+// 33.2; two 6144 x 2048 at 4 bpw, 1024 rows 979 -> 173.  In graph replays,
+// without the launches' host time (fp16 codebooks): 2048 x 6144 at 4 bpw, 3 /
+// 16 / 64 rows 25.3 / 26.7 / 36.3 -> 24.5 / 25.2 / 30.4; 6144 x 2048 24.2 /
+// 25.9 / 35.8 -> 22.4 / 22.8 / 27.2; 2048 x 2048 at 2 bpw, 16 rows 14.0 ->
+// 10.9.  Left behind them: 17 rows of 6144 x 6144 and 6144 x 4096 at 4 bpw (60.1
+// / 42.3 -> 62.3 / 43.3), 3 rows of the former (57.7 -> 58.4).  Bound by the gathers (13 us
 // of a 6144 x 2048 call at 4 bpw) and, below about a million codes, by the
 // two launches' latency (~12 us).
 //
@@ -64,14 +69,24 @@ constexpr int RW_PACK_MAX = ROT_ROW_MAX_T;
 constexpr int64_t RW_MAX_N = 8 * RW_PACK_MAX;
 constexpr int RW_CB_ROWS = 65536;
 // bf16 codebooks: up to this many rows are packed as two bf16 addends each,
-// which fit one 16-row tile, so the centroids need no rounding: exact, and
-// without the pass over the codebooks in every call.  Graph replays, us a
-// call, 8 rows, rounded / two addends (vq2_rht and vq2_gemm_small_m): 6144 x
-// 2048 at 4 bpw 25.5 / 23.3 (25.2), 2048 x 6144 27.5 / 26.1 (26.2), 2048 x
-// 2048 at 2 bpw 12.9 / 11.7 (13.6).  A second tile for 9 to 16 rows gains
-// less than it costs: 6144 x 2048 at 3 bpw, 16 rows 17.8 / 18.3.
+// which fit one 16-row tile, so the centroids need no rounding.  More rows
+// round them as gathered: rounding the codebooks first, in every call, cost up
+// to 4 us of it.  Graph replays, us a call, first / now (vq2_rht and
+// vq2_gemm_small_m before): 8 rows 6144 x 2048 at 4 bpw 25.5 / 22.8 (25.2),
+// 2048 x 6144 27.6 / 25.6 (26.3), 512 x 6144 19.9 / 16.2 (16.6); 17 rows 512 x
+// 2048 at 4 bpw 18.2 / 15.0 (15.4), 64 rows 6144 x 2048 at 3 bpw 22.0 / 21.1
+// (31.7).  Left behind the launches before: 9 to 17 rows of 512 x 6144 (9 rows
+// 17.5 / 17.1) and of 6144 x 4096 (43.1 / 41.4) at 4 bpw.
 constexpr int64_t RW_BF_ROWS = 8;
-static_assert(2 * RW_BF_ROWS <= 16, "both addends of every row in one row tile");
+static_assert(RW_BF_ROWS <= 8, "both addends of every row in one row tile");
+
+// fp32 codebooks: with one 16-bit stage and up to this many gathers they are
+// rounded as gathered, 32 bytes a code, else once per call by the packing
+// launch.  Graph replays, us a call, once per call / as gathered: 512 x 2048
+// at 2 bpw, 8 rows 13.8 / 12.1, 1024 x 2048 13.7 / 11.9; 17 rows 2048 x 6144
+// (1.5 M codes) 21.1 / 21.8; with two 16-bit stages 512 x 2048 15.5 / 16.8,
+// 6144 x 2048 24.6 / 31.2.
+constexpr int64_t RW_F32_GATHERS = 1 << 20;
 
 // ------------------------------------------------------------- the packing
 struct RowsPackArgs {
@@ -88,7 +103,7 @@ struct RowsPackArgs {
     float scale;
     int act_dt;  // type the rotated activation is rounded to first
     half8_t* a;  // packed activation
-    int bf;      // two bf16 addends a value, the second in row m + row
+    int bf;      // two bf16 addends a value, the second in row 8 + row of the one tile
     int* e;      // exponent of each row's scale
     uint32_t* cnt;  // arrival counters of the product, to be cleared
     int n_cnt;
@@ -108,6 +123,28 @@ __device__ __forceinline__ float rows_round_act(float v, int dt)
     return v;
 }
 
+__device__ __forceinline__ half8_t rows_bf16_to_half(u32x4 u)
+{
+    half8_t h;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        h[2 * k] = (_Float16)__uint_as_float(u[k] << 16);
+        h[2 * k + 1] = (_Float16)__uint_as_float(u[k] & 0xFFFF0000u);
+    }
+    return h;
+}
+
+__device__ __forceinline__ half8_t rows_f32_to_half(u32x4 lo, u32x4 hi)
+{
+    half8_t h;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        h[k] = (_Float16)__uint_as_float(lo[k]);
+        h[4 + k] = (_Float16)__uint_as_float(hi[k]);
+    }
+    return h;
+}
+
 // Centroid i of cb0, then cb1, rounded to fp16.
 __device__ __forceinline__ void rows_cvt_codebook(const RowsPackArgs& a, int64_t i)
 {
@@ -119,22 +156,8 @@ __device__ __forceinline__ void rows_cvt_codebook(const RowsPackArgs& a, int64_t
         dst = a.h1;
         if (i >= a.cb1_rows) return;
     }
-    half8_t h;
-    if (a.cb_dt == VQ2_DT_BF16) {
-        const u32x4 u = *((const u32x4*)src + i);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            h[2 * k] = (_Float16)__uint_as_float(u[k] << 16);
-            h[2 * k + 1] = (_Float16)__uint_as_float(u[k] & 0xFFFF0000u);
-        }
-    } else {
-        const u32x4 lo = *((const u32x4*)src + 2 * i), hi = *((const u32x4*)src + 2 * i + 1);
-#pragma unroll
-        for (int k = 0; k < 4; k++) {
-            h[k] = (_Float16)__uint_as_float(lo[k]);
-            h[4 + k] = (_Float16)__uint_as_float(hi[k]);
-        }
-    }
+    const half8_t h = a.cb_dt == VQ2_DT_BF16 ? rows_bf16_to_half(*((const u32x4*)src + i))
+                                             : rows_f32_to_half(*((const u32x4*)src + 2 * i), *((const u32x4*)src + 2 * i + 1));
     dst[i] = h;
 }
 
@@ -187,22 +210,22 @@ __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackAr
     for (int k = 0; k < 8; k++) h[k] = (_Float16)ldexpf(v[k], e);
     auto put = [&](int64_t r, half8_t w) { a.a[(((r >> 4) * a.kt + kt) * 8 + t) * 64 + q * 16 + (r & 15)] = w; };
     if (!a.bf) return put(row, h);
+    // the upper 8 of a value's 11 bits, and the rest (nothing of an infinity)
     u32x4 hi, lo;
 #pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const float f = (float)h[k];
-        const uint32_t b = f32_to_bf16_bits(f);
-        const uint32_t c = fabsf(f) < __builtin_inff() ? f32_to_bf16_bits(f - bf16_bits_to_f32(b)) : 0u;
-        if (k & 1) {
-            hi[k >> 1] |= b << 16;
-            lo[k >> 1] |= c << 16;
-        } else {
-            hi[k >> 1] = b;
-            lo[k >> 1] = c;
+    for (int k = 0; k < 4; k++) {
+        uint32_t u[2], r[2];
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float f = (float)h[2 * k + j];
+            u[j] = __float_as_uint(f) & 0xFFFF0000u;
+            r[j] = fabsf(f) < __builtin_inff() ? __float_as_uint(f - __uint_as_float(u[j])) : 0u;
         }
+        hi[k] = (u[0] >> 16) | u[1];
+        lo[k] = (r[0] >> 16) | (r[1] & 0xFFFF0000u);
     }
     put(row, __builtin_bit_cast(half8_t, hi));
-    put(a.m + row, __builtin_bit_cast(half8_t, lo));
+    put(8 + row, __builtin_bit_cast(half8_t, lo));
 }
 
 // ------------------------------------------------------------- the product
@@ -220,11 +243,10 @@ struct RowsArgs {
     const half8_t* a;  // packed activation
     const int* e;
     int m;
-    int mp;  // packed rows: m, with two bf16 addends 2 m
     int kt;  // k tiles
     int ng;
-    const half8_t* cb0;  // fp16 codebooks (rows_gemm_kernel<S2, MT, 1>: bf16)
-    const half8_t* cb1;
+    const void* cb0;  // codebooks (rows_wide_kernel: fp16)
+    const void* cb1;
     int s_dt;
     int y_dt;
     float rs;
@@ -262,6 +284,36 @@ struct RowCodes {
     }
 };
 
+// How rows_gemm_kernel takes its codebooks: the dtype codes (bf16 and fp32
+// rounded to fp16 as gathered), or bf16 as it is.
+constexpr int RW_CB_BF = 3;
+
+// A centroid as gathered, and as the matrix instruction's operand.
+template <int CB>
+struct RowCentroid {
+    half8_t h;
+    __device__ __forceinline__ void load(const void* cb, uint32_t code) { h = ((const half8_t*)cb)[code]; }
+    __device__ __forceinline__ half8_t operand() const { return h; }
+};
+
+template <>
+struct RowCentroid<VQ2_DT_BF16> {
+    u32x4 u;
+    __device__ __forceinline__ void load(const void* cb, uint32_t code) { u = ((const u32x4*)cb)[code]; }
+    __device__ __forceinline__ half8_t operand() const { return rows_bf16_to_half(u); }
+};
+
+template <>
+struct RowCentroid<VQ2_DT_F32> {
+    u32x4 lo, hi;
+    __device__ __forceinline__ void load(const void* cb, uint32_t code)
+    {
+        lo = ((const u32x4*)cb)[2 * (size_t)code];
+        hi = ((const u32x4*)cb)[2 * (size_t)code + 1];
+    }
+    __device__ __forceinline__ half8_t operand() const { return rows_f32_to_half(lo, hi); }
+};
+
 __device__ __forceinline__ const RowsSeg& rows_seg(const RowsArgs& a, int tile)
 {
     int s = 0;
@@ -275,10 +327,10 @@ constexpr int RW_WIDE_WAVES = 4; // waves of a rows_wide_kernel workgroup
 constexpr int RW_MAX_Z = 4;  // workgroups that share a tile's k tiles
 
 // Up to 16 * MT rows: a workgroup is nc column tiles of 16 columns x kw waves
-// over the k tiles; blockIdx.y counts blocks of 16 * MT rows.  BF: bf16
-// codebooks and packed rows, the addends of row r in rows r and m + r of the
-// one row block.
-template <int S2, int MT, int BF>
+// over the k tiles; blockIdx.y counts blocks of 16 * MT rows.  CB: the
+// codebooks (RowCentroid); with RW_CB_BF the packed rows are bf16 too, the
+// addends of row r in rows r and 8 + r of the one tile.
+template <int S2, int MT, int CB>
 __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const RowsArgs a)
 {
     touch_kernargs(a);
@@ -296,7 +348,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     const int mt0 = (int)blockIdx.y * MT;
     const half8_t zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     auto mfma = [](half8_t x, half8_t b, f32x4_t c) {
-        return mfma_16<!BF>(__builtin_bit_cast(u32x4, x), __builtin_bit_cast(u32x4, b), c);
+        return mfma_16<CB != RW_CB_BF>(__builtin_bit_cast(u32x4, x), __builtin_bit_cast(u32x4, b), c);
     };
 
     // what the epilogue needs, loaded ahead of everything else: the rows'
@@ -309,7 +361,7 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
 
     const int64_t rowoff = (int64_t)(col0 + nl < sg.rows ? col0 + nl : 0) * a.ng;
     // row tiles past the last one read tile mt_last again (results dropped)
-    const int mt_last = (a.mp - 1) >> 4;
+    const int mt_last = (a.m - 1) >> 4;
     const half8_t* ap[MT];
 #pragma unroll
     for (int i = 0; i < MT; i++) ap[i] = a.a + (int64_t)min(mt0 + i, mt_last) * a.kt * 512 + lane;
@@ -326,34 +378,49 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
     };
     if (k0 < a.kt) load_codes(k0);
     if constexpr (S2 == VQ2_S2_U8) {
-        for (int i = tid; i < 256; i += (int)blockDim.x) s_c1[i] = a.cb1[i];
+        for (int i = tid; i < 256; i += (int)blockDim.x) {
+            RowCentroid<CB> c;
+            c.load(a.cb1, i);
+            s_c1[i] = c.operand();
+        }
         __syncthreads();
     }
     for (int kt = k0; kt < a.kt; kt += kstep) {
         const bool g_ok = kt * RW_TILE_G + q * 8 < a.ng;
-        half8_t b0[8], b1[8];
+        // steps whose gathers are in flight together: as many as the 128 registers of a lane hold
+        constexpr int TS = CB == VQ2_DT_F32 || (CB == VQ2_DT_BF16 && S2 == VQ2_S2_U8 && MT >= 3) ? 4 : 8;
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            b0[t] = a.cb0[cd.c0(t)];
-            if constexpr (S2 == VQ2_S2_U16) b1[t] = a.cb1[cd.c1(t)];
-            if constexpr (S2 == VQ2_S2_U8) b1[t] = s_c1[cd.c1(t)];
-        }
-        if (kt + kstep < a.kt) load_codes(kt + kstep);
+        for (int t0 = 0; t0 < 8; t0 += TS) {
+            RowCentroid<CB> b0[TS];
+            RowCentroid<S2 == VQ2_S2_U8 ? VQ2_DT_F16 : CB> b1[TS];  // (16,8): from LDS, as operands
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            half8_t av[MT];
+            for (int t = 0; t < TS; t++) {
+                b0[t].load(a.cb0, cd.c0(t0 + t));
+                if constexpr (S2 == VQ2_S2_U16) b1[t].load(a.cb1, cd.c1(t0 + t));
+                if constexpr (S2 == VQ2_S2_U8) b1[t].h = s_c1[cd.c1(t0 + t)];
+            }
+            if (t0 + TS == 8 && kt + kstep < a.kt) load_codes(kt + kstep);
 #pragma unroll
-            for (int i = 0; i < MT; i++) av[i] = ap[i][((int64_t)kt * 8 + t) * 64];
-            const half8_t bb = g_ok ? b0[t] : zero8;
+            for (int t = 0; t < TS; t++) {
+                half8_t av[MT];
 #pragma unroll
-            for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bb, acc[i]);
-            if constexpr (S2 != VQ2_S2_NONE) {
-                const half8_t bc = g_ok ? b1[t] : zero8;
+                for (int i = 0; i < MT; i++) av[i] = ap[i][((int64_t)kt * 8 + t0 + t) * 64];
+                const half8_t bb = g_ok ? b0[t].operand() : zero8;
 #pragma unroll
-                for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bc, acc[i]);
+                for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bb, acc[i]);
+                if constexpr (S2 != VQ2_S2_NONE) {
+                    const half8_t bc = g_ok ? b1[t].operand() : zero8;
+#pragma unroll
+                    for (int i = 0; i < MT; i++) acc[i] = mfma(av[i], bc, acc[i]);
+                }
             }
         }
     }
+
+    // rows r and 8 + r of a tile lie 32 lanes apart: the sum of the two addends
+    if constexpr (CB == RW_CB_BF)
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc[0][e] += xor32(acc[0][e]);
 
     // D[i][j]: activation row 4 (l / 16) + e of the tile, column l % 16; the
     // waves' sums meet in LDS and are added in wave order
@@ -393,22 +460,15 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         __syncthreads();
         nred = 1;
     }
-    // the sum of the output at p, over the waves that shared its k tiles
-    auto total = [&](const float* p) {
-        float sum = 0.0f;
-        for (int w = 0; w < nred; w++) {
-            sum += p[w * TILE];
-            if constexpr (BF) sum += p[w * TILE + a.m * LD];
-        }
-        return sum;
-    };
     if (nc == 1) {
         // (blockDim is a multiple of 16: the thread's column stays)
         const int c = tid % 16;
         const float s = raw_as_f32(s_pre, a.s_dt);
         if (col0 + c >= sg.rows) return;
         for (int r = tid / 16; r < mrows; r += (int)blockDim.x / 16) {
-            const float sum = total(red + r * LD + c);
+            const float* p = red + r * LD + c;
+            float sum = 0.0f;
+            for (int w = 0; w < nred; w++) sum += p[w * TILE];
             store_from_f32(sg.y, a.y_dt, (int64_t)(mt0 * 16 + r) * sg.y_stride + col0 + c, (ldexpf(sum, -s_e[r]) * s) * a.rs);
         }
         return;
@@ -420,7 +480,9 @@ __global__ void __launch_bounds__(64 * RW_MAX_WAVES) rows_gemm_kernel(const Rows
         const RowsSeg& so = rows_seg(a, tl);
         const int col = (tl - so.tile0) * 16 + c;
         if (col >= so.rows) continue;
-        const float sum = total(red + ct * kw * TILE + r * LD + c);
+        const float* p = red + ct * kw * TILE + r * LD + c;
+        float sum = 0.0f;
+        for (int w = 0; w < nred; w++) sum += p[w * TILE];
         const float s = load_as_f32(so.scale, a.s_dt, col);
         store_from_f32(so.y, a.y_dt, (int64_t)(mt0 * 16 + r) * so.y_stride + col, (ldexpf(sum, -s_e[r]) * s) * a.rs);
     }
@@ -466,7 +528,7 @@ __global__ void __launch_bounds__(64 * RW_WIDE_WAVES, 2) rows_wide_kernel(const 
     };
     load_codes(c0, kt0);
     if constexpr (S2 == VQ2_S2_U8) {
-        for (int i = tid; i < 256; i += 64 * NW) s_c1[i] = a.cb1[i];
+        for (int i = tid; i < 256; i += 64 * NW) s_c1[i] = ((const half8_t*)a.cb1)[i];
         __syncthreads();
     }
 
@@ -490,8 +552,8 @@ __global__ void __launch_bounds__(64 * RW_WIDE_WAVES, 2) rows_wide_kernel(const 
     auto gather = [&](const RowCodes<S2>& c, int t0, half8_t (&g0)[TS], half8_t (&g1)[TS]) {
 #pragma unroll
         for (int j = 0; j < TS; j++) {
-            g0[j] = a.cb0[c.c0(t0 + j)];
-            if constexpr (S2 == VQ2_S2_U16) g1[j] = a.cb1[c.c1(t0 + j)];
+            g0[j] = ((const half8_t*)a.cb0)[c.c0(t0 + j)];
+            if constexpr (S2 == VQ2_S2_U16) g1[j] = ((const half8_t*)a.cb1)[c.c1(t0 + j)];
             if constexpr (S2 == VQ2_S2_U8) g1[j] = s_c1[c.c1(t0 + j)];
         }
     };
@@ -602,8 +664,8 @@ __global__ void __launch_bounds__(256) rows_sum_kernel(const RowsArgs a)
 
 // ------------------------------------------------------------------ launch
 struct RowsPlan {
-    int bf;            // bf16 products (RW_BF_ROWS)
-    int64_t mp;        // packed rows
+    int cb;            // codebooks of rows_gemm_kernel (RowCentroid)
+    int cvt;           // rounded to fp16 by the packing launch (cb = VQ2_DT_F16)
     int kt;
     int mt;            // 16-row tiles of a wave
     int kw, nc, nz;    // waves and workgroups over a column tile's k tiles; column tiles of a workgroup
@@ -661,13 +723,12 @@ static RowsPlan rows_plan(const RowsCall& c)
 {
     RowsPlan p{};
     p.kt = (int)((c.n / 8 + RW_TILE_G - 1) / RW_TILE_G);
-    p.bf = c.cb_dt == VQ2_DT_BF16 && c.m <= RW_BF_ROWS;
-    p.mp = p.bf ? 2 * c.m : c.m;
+    p.cb = c.cb_dt == VQ2_DT_BF16 && c.m <= RW_BF_ROWS ? RW_CB_BF : c.cb_dt;
     // row blocks of at most 64 rows, as even as whole tiles allow
-    const int64_t mtiles = (p.mp + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
+    const int64_t mtiles = (c.m + 15) / 16, blocks = (mtiles + RW_MAX_MT - 1) / RW_MAX_MT;
     p.mt = (int)((mtiles + blocks - 1) / blocks);
     for (int s = 0; s < c.nseg; s++) p.tiles += (c.seg[s].rows + 15) / 16;
-    p.grid_y = (p.mp + 16 * p.mt - 1) / (16 * p.mt);
+    p.grid_y = (c.m + 16 * p.mt - 1) / (16 * p.mt);
     // Few column tiles leave CUs idle, and a CU gathers at most ~0.9 codes a
     // ns however few others do: several workgroups then share a tile's k
     // tiles, while a workgroup has 6144 gathers or more (below that the
@@ -689,13 +750,17 @@ static RowsPlan rows_plan(const RowsCall& c)
     p.nc = (int)std::max<int64_t>(1, std::min<int64_t>(8 / p.kw, p.tiles * p.grid_y / device_cu_count()));
     if (c.m > 16 * RW_MAX_MT) rows_plan_wide(c, p);
     p.grid_x = (p.tiles + p.nc - 1) / p.nc;
-    const bool cvt = c.cb_dt != VQ2_DT_F16 && !p.bf;
+    int64_t codes = 0;
+    for (int s = 0; s < c.nseg; s++) codes += c.seg[s].rows * (c.n / 8);
+    p.cvt = c.cb_dt == VQ2_DT_BF16 ? p.wide
+            : c.cb_dt == VQ2_DT_F32 && (p.wide || c.s2 == VQ2_S2_U16 || codes * p.grid_y > RW_F32_GATHERS);
+    if (p.cvt) p.cb = VQ2_DT_F16;
     const int64_t units = p.nz > 1 && !p.wide ? p.grid_x * p.grid_y : 0;
     p.e = up256((size_t)units * sizeof(uint32_t));
     p.a = p.e + up256((size_t)c.m * sizeof(int));
-    p.h0 = p.a + (size_t)((p.mp + 15) / 16) * p.kt * 512 * sizeof(half8_t);
-    p.h1 = p.h0 + (cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
-    p.part = p.h1 + (!cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
+    p.h0 = p.a + (size_t)((c.m + 15) / 16) * p.kt * 512 * sizeof(half8_t);
+    p.h1 = p.h0 + (p.cvt ? (size_t)RW_CB_ROWS * sizeof(half8_t) : 0);
+    p.part = p.h1 + (!p.cvt || c.s2 == VQ2_S2_NONE ? 0 : (size_t)(c.s2 == VQ2_S2_U8 ? 256 : RW_CB_ROWS) * sizeof(half8_t));
     p.total = p.part + (p.wide && p.nz > 1 ? (size_t)p.nz * c.m * p.tiles * 16 : (size_t)units * p.nz * 256 * p.mt) *
                            sizeof(float);
     return p;
@@ -719,7 +784,7 @@ size_t rows_workspace_bytes(const RowsCall& c)
     return rows_check(c) == VQ2_OK ? rows_plan(c).total : 0;
 }
 
-template <int S2, int MT, int BF = 0>
+template <int S2, int MT, int CB>
 static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
     // opt in to more than 64 KiB of dynamic LDS, once per instantiation
@@ -727,24 +792,41 @@ static hipError_t rows_launch_t(const RowsArgs& a, dim3 grid, int waves, hipStre
     static hipError_t attr = hipSuccess;
     constexpr size_t SHM_WAVE = 16 * MT * 17 * sizeof(float);
     std::call_once(once, [] {
-        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT, BF>,
+        attr = hipFuncSetAttribute((const void*)rows_gemm_kernel<S2, MT, CB>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)(RW_MAX_WAVES * SHM_WAVE));
     });
     if (attr != hipSuccess) return attr;
     const size_t shm = waves * SHM_WAVE;
-    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT, BF>), grid, dim3(64 * waves), shm, st, a);
+    hipLaunchKernelGGL((rows_gemm_kernel<S2, MT, CB>), grid, dim3(64 * waves), shm, st, a);
     return hipGetLastError();
 }
 
-template <int S2>
-static hipError_t rows_launch_s(int mt, int bf, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
+template <int S2, int CB>
+static hipError_t rows_launch_c(int mt, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
 {
-    if (bf) return rows_launch_t<S2, 1, 1>(a, grid, waves, st);
-    switch (mt) {
-    case 1: return rows_launch_t<S2, 1>(a, grid, waves, st);
-    case 2: return rows_launch_t<S2, 2>(a, grid, waves, st);
-    case 3: return rows_launch_t<S2, 3>(a, grid, waves, st);
-    default: return rows_launch_t<S2, 4>(a, grid, waves, st);
+    if constexpr (CB == RW_CB_BF) {
+        return rows_launch_t<S2, 1, CB>(a, grid, waves, st);
+    } else {
+        switch (mt) {
+        case 1: return rows_launch_t<S2, 1, CB>(a, grid, waves, st);
+        case 2: return rows_launch_t<S2, 2, CB>(a, grid, waves, st);
+        case 3: return rows_launch_t<S2, 3, CB>(a, grid, waves, st);
+        default: return rows_launch_t<S2, 4, CB>(a, grid, waves, st);
+        }
+    }
+}
+
+template <int S2>
+static hipError_t rows_launch_s(int mt, int cb, const RowsArgs& a, dim3 grid, int waves, hipStream_t st)
+{
+    switch (cb) {
+    case VQ2_DT_F16: return rows_launch_c<S2, VQ2_DT_F16>(mt, a, grid, waves, st);
+    case VQ2_DT_BF16: return rows_launch_c<S2, VQ2_DT_BF16>(mt, a, grid, waves, st);
+    case RW_CB_BF: return rows_launch_c<S2, RW_CB_BF>(mt, a, grid, waves, st);
+    default:
+        // fp32: rows_plan gathers only single 16-bit stages of it
+        if constexpr (S2 != VQ2_S2_U16) return rows_launch_c<S2, VQ2_DT_F32>(mt, a, grid, waves, st);
+        else return hipErrorInvalidValue;
     }
 }
 
@@ -802,7 +884,6 @@ int rows_launch(const RowsCall& c)
         return set_error(VQ2_ERR_ARG, "vq2_rows_gemm: workspace of %zu bytes (256-byte aligned) needed, got %zu", p.total,
                          c.ws_bytes);
     char* ws = (char*)c.workspace;
-    const bool cvt = c.cb_dt != VQ2_DT_F16 && !p.bf;
     hipStream_t st = (hipStream_t)c.stream;
 
     RowsPackArgs k{};
@@ -819,11 +900,11 @@ int rows_launch(const RowsCall& c)
     k.scale = c.xscale;
     k.act_dt = c.act_dt;
     k.a = (half8_t*)(ws + p.a);
-    k.bf = p.bf;
+    k.bf = p.cb == RW_CB_BF;
     k.e = (int*)(ws + p.e);
     k.cnt = (uint32_t*)ws;
     k.n_cnt = p.nz > 1 && !p.wide ? (int)(p.grid_x * p.grid_y) : 0;
-    if (cvt) {
+    if (p.cvt) {
         k.cb0 = c.cb0;
         k.cb1 = c.cb1;
         k.cb_dt = c.cb_dt;
@@ -838,11 +919,10 @@ int rows_launch(const RowsCall& c)
     a.a = k.a;
     a.e = k.e;
     a.m = (int)c.m;
-    a.mp = (int)p.mp;
     a.ng = (int)(c.n / 8);
     a.kt = p.kt;
-    a.cb0 = cvt ? k.h0 : (const half8_t*)c.cb0;
-    a.cb1 = cvt ? k.h1 : (const half8_t*)c.cb1;
+    a.cb0 = p.cvt ? k.h0 : c.cb0;
+    a.cb1 = p.cvt ? k.h1 : c.cb1;
     a.s_dt = c.s_dt;
     a.y_dt = c.y_dt;
     a.rs = c.rs;
@@ -875,9 +955,9 @@ int rows_launch(const RowsCall& c)
         return VQ2_OK;
     }
     switch (c.s2) {
-    case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
-    case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
-    default: err = rows_launch_s<VQ2_S2_NONE>(p.mt, p.bf, a, grid, p.kw * p.nc, st); break;
+    case VQ2_S2_U8: err = rows_launch_s<VQ2_S2_U8>(p.mt, p.cb, a, grid, p.kw * p.nc, st); break;
+    case VQ2_S2_U16: err = rows_launch_s<VQ2_S2_U16>(p.mt, p.cb, a, grid, p.kw * p.nc, st); break;
+    default: err = rows_launch_s<VQ2_S2_NONE>(p.mt, p.cb, a, grid, p.kw * p.nc, st); break;
     }
     if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm launch");
     return VQ2_OK;

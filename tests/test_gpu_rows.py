@@ -64,6 +64,19 @@ def _check(y, xr, m, cb0, cb1, rs=1.0):
     (270, 5003, 512, 512, 3, torch.float32, torch.float16, torch.float32),
     (400, 5003, 512, 512, 2, torch.float16, torch.float32, torch.float16),
     (193, 3100, 1024, 1024, 4, torch.float16, torch.float16, torch.float32),
+    # codebooks rounded as gathered (bf16 from 9 rows on, with fewer steps in
+    # flight from 33 on at 3 bpw; fp32 with one 16-bit stage), and fp32 ones
+    # of two such stages or more than 2^20 gathers
+    (8, 77, 320, 64, 3, torch.float16, torch.bfloat16, torch.float32),
+    (9, 77, 320, 64, 2, torch.float16, torch.bfloat16, torch.float32),
+    (20, 130, 2048, 2048, 4, torch.bfloat16, torch.bfloat16, torch.bfloat16),
+    (33, 65, 1024, 1024, 3, torch.float16, torch.bfloat16, torch.float32),
+    (64, 33, 320, 64, 3, torch.float32, torch.bfloat16, torch.float32),
+    (50, 600, 2048, 2048, 4, torch.float32, torch.bfloat16, torch.float32),
+    (5, 700, 1024, 1024, 3, torch.float16, torch.float32, torch.float32),
+    (40, 129, 320, 64, 2, torch.float32, torch.float32, torch.float32),
+    (6, 129, 512, 512, 4, torch.float32, torch.float32, torch.float32),
+    (3, 2200, 4096, 4096, 2, torch.float16, torch.float32, torch.float32),
 ])
 def test_rows_gemm_vs_oracle(dev, M, rows, n, hb, bpw, x_dtype, cb_dtype, y_dtype):
     seed = 9900 + M
