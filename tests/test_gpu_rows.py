@@ -57,7 +57,8 @@ def _check(y, xr, m, cb0, cb1, rs=1.0):
     (65, 2048, 6144, 2048, 2, torch.float16, torch.bfloat16, torch.float32),  # row blocks of 64 and 1
     (100, 700, 2048, 2048, 4, torch.float16, torch.float16, torch.float32),
     # 128 and 256 rows a workgroup: remainders of the row and column blocks, a
-    # short last k tile, the k tiles in one, two and four shares of either
+    # short last k tile, k tiles in one, two and four shares (every plan of
+    # either: test_rows_gemm_plans)
     (129, 5003, 576, 64, 2, torch.float16, torch.float16, torch.float16),
     (65, 6001, 2048, 2048, 2, torch.bfloat16, torch.float16, torch.float32),
     (65, 3100, 2048, 2048, 4, torch.bfloat16, torch.bfloat16, torch.float32),
@@ -96,6 +97,44 @@ def test_rows_gemm_vs_oracle(dev, M, rows, n, hb, bpw, x_dtype, cb_dtype, y_dtyp
     _check(y, K.vq_rht(x, None, None, hb, out_dtype=torch.float32).cpu().numpy(), m, cb0, cb1)
     (y,) = K.vq_rows_gemm(x, mats, c0, c1, n, hb=0, rs=0.25, out_dtype=torch.float32)
     _check(y, x.float().cpu().numpy(), m, cb0, cb1, rs=0.25)
+
+
+# The launch plans of 256 CUs (rows_plan), one case each: rows a workgroup,
+# shares of the k tiles; column tiles a workgroup
+@pytest.mark.parametrize("M,rows,n,bpw,cb_dtype", [
+    # rows_wide_kernel, the last k tile short in all, shares of unequal k tiles in those of two or four
+    (129, (6001,), 320, 2, torch.float16),               # 128 rows, 1 share
+    (65, (6001,), 2240, 2, torch.float16),               # 2: 4 and 5 of 9 k tiles
+    (65, (5003,), 3136, 3, torch.bfloat16),              # 4 of 13
+    (65, (6001,), 1600, 4, torch.float16),               # 2 of 7
+    (65, (3000,), 2240, 4, torch.float32),               # 4 of 9
+    (129, (12300,), 320, 3, torch.float16),              # 256 rows, 1 share
+    (129, (8200,), 2240, 3, torch.float16),              # 2 of 9
+    (129, (3000,), 3136, 2, torch.bfloat16),             # 4 of 13
+    (129, (3000,), 1600, 4, torch.float16),              # 4 of 7
+    (257, (3000,), 1600, 4, torch.float16),              # 2 of 7
+    (300, (2040, 1000, 20), 2240, 3, torch.float16),     # three matrices
+    # rows_gemm_kernel, several column tiles a workgroup: the last workgroup's past the last
+    # matrix, one matrix's tiles beside the next one's
+    (3, (8201,), 512, 2, torch.float16),                 # 2 column tiles, 2 waves each
+    (8, (16500,), 320, 2, torch.bfloat16),               # 4, two bf16 addends a value
+    (20, (8000, 300, 17), 256, 3, torch.bfloat16),       # 2
+    (64, (12300,), 64, 4, torch.float16),                # 3
+    (100, (8200, 33), 128, 4, torch.float32),            # 4, two row blocks
+    (200, (8201,), 64, 3, torch.float16),                # 8, four row blocks
+])
+def test_rows_gemm_plans(dev, M, rows, n, bpw, cb_dtype):
+    seed = 9700 + M
+    ms = [synth.vq_matrix(seed + i, r, n, bpw=bpw) for i, r in enumerate(rows)]
+    cb0, cb1 = _books(seed + 10, bpw, cb_dtype)
+    x = synth.activations(seed + 12, (M, n), dtype=torch.float32).to(dev)
+    mats = [tuple(_on(dev, m["idx0"], m["idx1"], m["scale"])) + (r,) for m, r in zip(ms, rows)]
+    ys = K.vq_rows_gemm(x, mats, *_on(dev, cb0, cb1), n, hb=0)
+    xr = fp16_row_scaled(x.cpu().numpy())
+    h0, h1 = cb0.half(), None if cb1 is None else cb1.half()
+    for y, m in zip(ys, ms):
+        ref = O.np_gemv64(xr, m["idx0"], m["idx1"], h0, h1, m["scale"])
+        assert np.all(np.abs(y.cpu().numpy() - ref) <= TOL_SUM * np.abs(ref).max(1, keepdims=True))
 
 
 def test_rows_gemm_unaligned_rows_row_scales_and_nan(dev):
