@@ -15,7 +15,6 @@ import torch
 
 from compressai_amd import kernels as K, synth
 from compressai_amd.moe import MoELayer, ResidentMoEExperts
-from compressai_amd.rot import Rot
 from oracle import vq2_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -98,6 +97,28 @@ def test_ids_outside_the_pool_poison_their_token_alone(dev):
     assert bool(torch.isnan(out[rows]).all())
     keep = [t for t in range(T) if t not in (3, 7, 39)]
     assert torch.equal(out[keep], good[keep])
+
+
+def test_more_pairs_than_the_sorting_workgroup_holds_in_registers(dev):
+    """Above 5120 pairs (256 threads, 20 ids each) the pairs are sorted in
+    several batches, their ids read again in the second pass: every token's
+    result is the one that a call of few tokens gives, bit for bit (it depends
+    on the token's own pairs alone), tokens with ids outside the pool NaN."""
+    E, T, P, H, I = 9, 1811, 3, 512, 64  # 5433 pairs
+    gu, gus, dn, dns = _pools(9910, E, H, I)
+    args = [t.to(dev) for t in (gu, gus, dn, dns)]
+    cb = synth.codebook(9915).to(dev)
+    th, ti = _tables(H, H, 9916, dev), _tables(I, I, 9918, dev)
+    h = synth.activations(9920, (T, H)).to(dev)
+    ids = torch.randint(0, E, (T, P), generator=synth.gen(9921))
+    ids[5, 1], ids[1700, 0], ids[1810, 2] = E, -1, E + 7
+    ids, w = ids.to(dev), torch.rand(T, P, generator=synth.gen(9922)).to(dev)
+    call = lambda t0, t1: K.vq_moe_rows(h[t0:t1], ids[t0:t1], w[t0:t1], *args, cb, th[0], ti[0])
+    out = call(0, T)
+    parts = torch.cat([call(t, min(T, t + 600)) for t in range(0, T, 600)])
+    bad = torch.zeros(T, dtype=torch.bool, device=dev)
+    bad[[5, 1700, 1810]] = True
+    assert bool(torch.isnan(out[bad]).all()) and torch.equal(out[~bad], parts[~bad])
 
 
 @pytest.mark.parametrize("cb_dtype", [torch.float16, torch.bfloat16])
