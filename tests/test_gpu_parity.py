@@ -657,8 +657,8 @@ def test_gemm_small_m_split_sum_in_launch_is_deterministic(dev):
 
 @pytest.mark.parametrize("B", [3, 70])
 def test_packed_linear_small_m_path(dev, B):
-    """PackedLinear at batch >= 3 (matrix-core GEMM, chunked at 64 rows)
-    against the fp64 oracle of RHT + VQ GEMV."""
+    """PackedLinear at batch >= 3 (all rows in one matrix-core product,
+    vq_rows_gemm) against the fp64 oracle of RHT + VQ GEMV."""
     from compressai_amd.runtime import PackedLinear
     out, n = 512, 2048
     m = synth.vq_matrix(7400, out, n, bpw=4)
@@ -669,6 +669,24 @@ def test_packed_linear_small_m_path(dev, B):
     xr = O.rht(x, lin.rot.perm.cpu(), lin.rot.sign.float().cpu().numpy().astype(np.int8), lin.rot.hb)
     _, y64 = O.vq_gemv(xr.astype(np.float32), m["idx0"], m["idx1"], cbs["16"].cpu(), cbs["16_16"].cpu(),
                        lin.scale.cpu())
+    assert y.shape == (B, out)
+    assert _rowwise_err(y, y64) < TOL
+
+
+@pytest.mark.parametrize("B", [3, 70, 129])
+def test_packed_linear_wider_than_the_row_product(dev, B):
+    """Rows of more than 8192 values: the rotation, then vq_gemm_small_m in
+    chunks of 64 rows, the last one short."""
+    from compressai_amd.runtime import PackedLinear
+    out, n = 96, 10240
+    m = synth.vq_matrix(7410, out, n, bpw=2)
+    cbs = {"16": synth.codebook(7411).to(dev)}
+    lin = PackedLinear((out, n), (16,), "t_wide", [m["idx0"]], m["scale"], cbs, dev)
+    assert n > K.ROWS_GEMM_MAX_N
+    x = synth.activations(7414, (B, n), dtype=torch.float32)
+    y = lin(x.to(dev), out_dtype=torch.float32).cpu().numpy()
+    xr = O.rht(x, lin.rot.perm.cpu(), lin.rot.sign.float().cpu().numpy().astype(np.int8), lin.rot.hb)
+    _, y64 = O.vq_gemv(xr.astype(np.float32), m["idx0"], None, cbs["16"].cpu(), None, lin.scale.cpu())
     assert y.shape == (B, out)
     assert _rowwise_err(y, y64) < TOL
 
