@@ -2,9 +2,8 @@
 
 The library and ``_vq2_host`` (the native argument checks and launches of the
 entries that small calls spend their time in, csrc/vq2_host.cpp) are built
-in-tree (``python -m compressai_amd.build`` or
-``__graft_entry__.build()``) and loaded from this package directory.  There is
-no fallback: if the library is missing, every entry raises.
+in-tree (``__graft_entry__.build()``) and loaded from this package directory.
+There is no fallback: if either is missing, the entries that need it raise.
 """
 from __future__ import annotations
 

@@ -9,10 +9,12 @@
 // reference-layout pools.  The one-pair kernels (vq2_sorted_moe.hip) gather an
 // expert's codes once per pair, ~0.8 us each; a prompt's chunk of 512 tokens
 // has 18 pairs an expert.  Here the pairs are grouped by expert and a
-// workgroup multiplies up to 32 or 64 of them by 128 rows of the expert, so a layer
-// costs one pass over the experts' codes whatever the tokens: bound by the
-// gathers, 101 M codes a layer of 257 experts at the ~240 G/s that the L2s
-// serve = 0.42 ms.  Five launches:
+// workgroup multiplies up to 32 or 64 of them by 128 rows of the expert, so an
+// expert's codes are gathered once per such tile: at least one per expert
+// that has pairs, and ceil(T / tile) for one that every token names, as the
+// shared expert.  Bound by those gathers: 393 K codes a tile at the ~240 G/s that
+// the L2s serve, 0.45 ms for the ~275 tiles of 512 tokens over 257 experts.
+// Five launches:
 //  1. moe_prep: workgroup 0 sorts the pairs by expert (a slot each) and cuts
 //     them into tiles; the others rotate a token each and pack it.
 //  2. moe_gemm, gate_up: gu[slot] = row sums * row scale, fp32.
@@ -34,9 +36,9 @@
 // 7e-7.
 //
 // Measured (35B shape, us a layer, router included, one-pair kernels before):
-// 72 tokens 521 -> 493, 128 tokens 896 -> 509, 512 tokens 3526 -> 590; at 512
-// tokens gate_up gathers 67 M codes in 0.37 ms, down 34 M in 0.2 (with all
-// codes alike 0.17 and 0.12).
+// 73 tokens 510 -> 462, 128 tokens 883 -> 489, 512 tokens 3432 -> 574 (graph
+// replays; bf16 codebook 561); at 512 tokens gate_up takes 0.35 ms, down 0.2
+// (with all codes alike 0.17 and 0.12).
 #include <algorithm>
 #include <mutex>
 
@@ -106,7 +108,7 @@ struct MoePackArgs {
     const int8_t* sign;
     float scale;
     u32x4* a;  // packed rows
-    int* e;    // their exponents (NS = 2)
+    int* e;    // their exponents (F16)
 };
 
 struct MoePlanArgs {
@@ -272,12 +274,12 @@ __global__ void __launch_bounds__(ROT_ROW_MAX_T) moe_act_kernel(const MoePackArg
 // ------------------------------------------------------------- the product
 struct MoeGemmArgs {
     const u32x4* a;      // packed rows
-    const int* e;        // their exponents (NS = 2)
+    const int* e;        // their exponents (F16)
     const int* row_of;   // packed row of a slot (null: the slot)
     const MoeTile* tiles;
     const int* n_tiles;
     const int16_t* idx;  // pool [n_experts, rows, ng]
-    const u32x4* cb;     // fp16 (NS = 2) or bf16 (NS = 3) codebook
+    const u32x4* cb;     // fp16 (F16) or bf16 codebook
     const void* scale;   // [n_experts, rows]
     int s_dt;
     int rows;
@@ -468,7 +470,8 @@ static MoeRowsPlan moe_rows_plan(const MoeRowsCall& c)
     p.pairs = c.tokens * c.P;
     // every expert may end with a short tile
     // 64 pairs a tile from 28 an expert on (35B shape, us a layer at 32 / 64
-    // pairs: 512 tokens, 18 an expert 610 / 777; 1024 tokens 939 / 846; 2048
+    // pairs when the line was set, before the router and the sorting took 20
+    // us less: 512 tokens, 18 an expert 610 / 777; 1024 tokens 939 / 846; 2048
     // tokens 1533 / 1333)
     p.mt = p.pairs >= 28 * c.n_experts ? 4 : 2;
     p.max_tiles = p.pairs / (16 * p.mt) + std::min<int64_t>(p.pairs, c.n_experts);

@@ -63,7 +63,11 @@ __device__ __forceinline__ float router_shared_weight(const void* gate, int g_dt
                                                       int64_t hidden, int lane)
 {
     // every pair of types with its loads in flight together (a loop over
-    // run-time types took 20 us a wave: fp16 gate, bf16 activation)
+    // run-time types took 20 us a wave: fp16 gate, bf16 activation).  Inlined
+    // into the one-launch MoE the nine cases spill 125 SGPRs where three and
+    // that loop spilled 76, at no cost: graph replays at the 35B shape, 1 / 8
+    // tokens 22.6 / 62.1 us either way with an fp16 activation, 30.1 / 62.0 ->
+    // 21.5 / 59.9 with a bf16 one.
     auto with_h = [&](auto gt) {
         constexpr int G = decltype(gt)::value;
         return h_dt == VQ2_DT_F16    ? router_gate_dot<G, VQ2_DT_F16>(gate, h, t, hidden, lane)

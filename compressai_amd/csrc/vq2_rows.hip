@@ -685,12 +685,16 @@ static size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 // per workgroup of 64 (rows_wide_kernel).  Rates in requests a ns, measured
 // (MI355X): rows_gemm_kernel 235; rows_wide_kernel a workgroup 1.0 with 128
 // rows and 0.75 with 256, all of them 200 and 160; nz > 1 adds the partials'
-// launch (4 us) and their traffic (5 TB/s).  Over nine shapes and 65 to 1024
-// rows the choice is within 10 % of the fastest of the seven (us a call, rows
-// x n, bits, activation rows: rows_gemm / chosen): 2 x 6144 x 2048, 4, 100
-// rows 77 / 53, 1024 rows 545 / 196; 2048 x 6144, 4, 256 rows 83 / 61, 1024
-// 299 / 124; three of 1024 x 2048, 2, 333 rows 45 / 39, 1024 103 / 59; 512 x
-// 2048, 2, stays (1024 rows 31.5, the best wide plan 35).
+// launch (4 us) and their traffic (5 TB/s).  It serves to order the plans, not
+// to tell their times: a CU with less than two workgroups and the rows that
+// pad a tile are not in it (2048 + 512 + 512 rows x 2048, 2, 333 rows: 21 us
+// for a launch of 33).  Over fourteen shapes and 70 to 1024 rows the choice
+// is the fastest of the seven or within 1 % of it (graph replays, us a call,
+// rows x n, bits, activation rows: rows_gemm / chosen / the next best): 2 x
+// 6144 x 2048, 4, 100 rows 73 / 53 / 56, 1024 rows 523 / 175 / 231; 2048 x
+// 6144, 4, 256 rows 81 / 59 / 62, 1024 297 / 118 / 118; 2048 + 512 + 512 x
+// 2048, 2, 333 rows 41.8 / 39.7 / 40.0; 2999 x 4096, 2, 100 rows 34.1 / 33.2 /
+// 36.1; 512 x 2048, 2, stays (1024 rows 29.3, the best wide plan 34.5).
 static void rows_plan_wide(const RowsCall& c, RowsPlan& p)
 {
     const double stages = c.s2 == VQ2_S2_U16 ? 2 : 1, m = (double)c.m;

@@ -1080,12 +1080,16 @@ def moe_rows_faster(pairs, n_experts, hidden, inter) -> bool:
     """Whether vq_moe_rows takes less time than the one-pair kernels: those
     gather ~480 codes a ns for each pair, it ~200 a ns for each expert of the
     pool (all touched at worst) behind ~30 us of launches.  Measured on MI355X
-    at the 35B shape (257 pool entries, 9 pairs a token, us a layer, one-pair
-    against grouped): 56 tokens 414 / 458, 64 471 / 471, 72 521 / 493, 128
-    896 / 509, 512 3526 / 609; the line lies at 73 tokens there.  Small pools
-    switch from MOE_ROWS_MIN_PAIRS pairs on (17 entries, 5 pairs a token, 52
-    tokens 246 / 82); fewer pairs stay on the one-pair kernels, as decode
-    batches do at the 35B shape."""
+    at the 35B shape (257 pool entries, 9 pairs a token, graph replays, us a
+    layer, one-pair against grouped): 56 tokens 392 / 404, 60 427 / 410, 72
+    504 / 449, 128 883 / 489, 512 3432 / 574; the line lies at 73 tokens
+    there.  Small pools switch from MOE_ROWS_MIN_PAIRS pairs on (17 entries, 5
+    pairs a token, 52 tokens 249 / 84); fewer pairs stay on the one-pair
+    kernels, as decode batches do at the 35B shape.  The line errs to that side:
+    the constants are older than the grouped path's present launches, which
+    are ahead from 58 tokens on at the 35B shape and, in the small pool, from
+    26 (133 / 83); past the line they were ahead in every shape measured (9 to
+    257 entries, hidden 512 to 4096)."""
     codes = 3 * hidden * inter // 8
     return pairs >= MOE_ROWS_MIN_PAIRS and pairs * codes / 480e3 > n_experts * codes / 200e3 + 30.0
 

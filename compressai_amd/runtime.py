@@ -61,12 +61,12 @@ SORTED_MIN_LAUNCH_CODES = SORTED_MIN_CODES
 #  * PackedProjections at batch 2 with SORTED_BATCH2_LAUNCH_MIN_CODES codes or
 #    more (gate + up: 24.6 against 37.6 in one gather-kernel launch).
 # Not used where it was slower: one 6144 x 2048 4 bpw matrix at batch 2
-# (23.2 against 20.9) and 3-4 (32-35 against 25 in vq_rows_gemm), the
-# down matrix at batch 3-4 (35-39 against 28), q / k / v at batch 2 (17.6
-# against 12.9; 0.79 M codes), projections of one activation at batch 3-4
-# (three of 1024 x 2048 22.0-24.4 against 13.6 in vq_rows_gemm, gate + up
-# 40.1-42.0 against 39.1): there it only serves released planes and rows too
-# wide for vq_rows_gemm.
+# (23.2 against 20.9) and 3-4 (32-35 against 22.4 in vq_rows_gemm; vq_rht and
+# vq_gemm_small_m 24.3), the down matrix at batch 3-4 (35-39 against 24.5;
+# 25.3), q / k / v at batch 2 (17.6 against 12.9; 0.79 M codes), projections of
+# one activation at batch 3-4 (q, k, v 20.2-21.2 against 11.9 in vq_rows_gemm,
+# gate + up 40.2-41.9 against 35.4): there it only serves released planes and
+# rows too wide for vq_rows_gemm.
 SORTED_BATCH = True
 SORTED_BATCH_MIN_CODES = 8 << 20
 # PackedProjections at batch 2 on the sorted layout from this many codes on
