@@ -103,7 +103,6 @@ struct RowsPackArgs {
     float scale;
     int act_dt;  // type the rotated activation is rounded to first
     half8_t* a;  // packed activation
-    int bf;      // two bf16 addends a value, the second in row 8 + row of the one tile
     int* e;      // exponent of each row's scale
     uint32_t* cnt;  // arrival counters of the product, to be cleared
     int n_cnt;
@@ -161,7 +160,9 @@ __device__ __forceinline__ void rows_cvt_codebook(const RowsPackArgs& a, int64_t
     dst[i] = h;
 }
 
-// Workgroup b < m: row b, one thread per group (vq2_rot_row.hpp).
+// Workgroup b < m: row b, one thread per group (vq2_rot_row.hpp).  BF: two
+// bf16 addends a value, the second in row 8 + b of the one tile.
+template <int BF>
 __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackArgs a)
 {
     extern __shared__ __align__(16) float s_x[];  // the row; later the exchanges
@@ -209,7 +210,10 @@ __global__ void __launch_bounds__(RW_PACK_MAX) rows_pack_kernel(const RowsPackAr
 #pragma unroll
     for (int k = 0; k < 8; k++) h[k] = (_Float16)ldexpf(v[k], e);
     auto put = [&](int64_t r, half8_t w) { a.a[(((r >> 4) * a.kt + kt) * 8 + t) * 64 + q * 16 + (r & 15)] = w; };
-    if (!a.bf) return put(row, h);
+    if constexpr (!BF) {
+        put(row, h);
+        return;
+    }
     // the upper 8 of a value's 11 bits, and the rest (nothing of an infinity)
     u32x4 hi, lo;
 #pragma unroll
@@ -856,13 +860,14 @@ static hipError_t rows_wide_s(int mt, const RowsArgs& a, dim3 grid, hipStream_t 
     return mt == 8 ? rows_wide_t<S2, 8, 4>(a, grid, st) : rows_wide_t<S2, 16, 2>(a, grid, st);
 }
 
-static hipError_t rows_pack_launch(const RowsPackArgs& p, hipStream_t st)
+static hipError_t rows_pack_launch(const RowsPackArgs& p, int bf, hipStream_t st)
 {
     const int T = std::max(64, (p.kt * RW_TILE_G + 63) / 64 * 64);
     int64_t blocks = p.m;
     if (p.cb0) blocks += (RW_CB_ROWS + p.cb1_rows + T - 1) / T;
     const size_t shm = (size_t)T * 8 * sizeof(float);
-    hipLaunchKernelGGL(rows_pack_kernel, dim3((unsigned)blocks), dim3(T), shm, st, p);
+    if (bf) hipLaunchKernelGGL(rows_pack_kernel<1>, dim3((unsigned)blocks), dim3(T), shm, st, p);
+    else hipLaunchKernelGGL(rows_pack_kernel<0>, dim3((unsigned)blocks), dim3(T), shm, st, p);
     return hipGetLastError();
 }
 
@@ -904,7 +909,6 @@ int rows_launch(const RowsCall& c)
     k.scale = c.xscale;
     k.act_dt = c.act_dt;
     k.a = (half8_t*)(ws + p.a);
-    k.bf = p.cb == RW_CB_BF;
     k.e = (int*)(ws + p.e);
     k.cnt = (uint32_t*)ws;
     k.n_cnt = p.nz > 1 && !p.wide ? (int)(p.grid_x * p.grid_y) : 0;
@@ -916,7 +920,7 @@ int rows_launch(const RowsCall& c)
         k.h0 = (half8_t*)(ws + p.h0);
         k.h1 = (half8_t*)(ws + p.h1);
     }
-    hipError_t err = rows_pack_launch(k, st);
+    hipError_t err = rows_pack_launch(k, p.cb == RW_CB_BF, st);
     if (err != hipSuccess) return set_hip_error(err, "vq2_rows_gemm packing launch");
 
     RowsArgs a{};

@@ -93,7 +93,9 @@ def vq_matmul(xr, i0, i1, cb0, cb1, scale, out, n, out_dtype, y=None):
 
 def _rows_ok(x2, n, rot):
     """Whether x2 [B, n] takes vq_rows_gemm (rotation and product of all rows
-    in two launches): three rows or more of a width its packing holds."""
+    in two launches): three rows or more of a width its packing holds.  It is
+    ahead of vq_rht and vq_gemm_small_m in eager calls, which the launches
+    bound, and in graph replays, but for a few sizes (csrc/vq2_rows.hip)."""
     return x2.shape[0] >= 3 and n % 64 == 0 and n <= K.ROWS_GEMM_MAX_N and rot.hb >= 64
 
 
