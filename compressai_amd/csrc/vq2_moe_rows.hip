@@ -13,7 +13,7 @@
 // expert's codes are gathered once per such tile: at least one per expert
 // that has pairs, and ceil(T / tile) for one that every token names, as the
 // shared expert.  Bound by those gathers: 393 K codes a tile at the ~240 G/s that
-// the L2s serve, 0.45 ms for the ~275 tiles of 512 tokens over 257 experts.
+// the L2s serve, 0.45 ms for the 272 tiles of 512 tokens over 257 experts.
 // Five launches:
 //  1. moe_prep: workgroup 0 sorts the pairs by expert (a slot each) and cuts
 //     them into tiles; the others rotate a token each and pack it.
