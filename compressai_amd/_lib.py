@@ -27,6 +27,7 @@ _vp, _i64, _i32, _f32 = ctypes.c_void_p, ctypes.c_int64, ctypes.c_int, ctypes.c_
 # argument types of every exported entry, in header order
 SIGNATURES = {
     "vq2_version": ([], _i32),
+    "vq2_stream_capture_id": ([_vp], _i64),
     "vq2_last_error": ([], ctypes.c_char_p),
     "vq2_gemv": ([_vp, _i32, _i64, _i64, _vp, _vp, _i32, _vp, _vp, _i32, _vp, _i32, _vp, _i32, _i64,
                   _i64, _i64, _f32, _vp], _i32),

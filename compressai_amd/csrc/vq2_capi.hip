@@ -74,6 +74,19 @@ extern "C" {
 
 int vq2_version(void) { return 100; }
 
+int64_t vq2_stream_capture_id(void* stream)
+{
+    // (the null stream cannot be captured, and asking it during a capture is an error)
+    if (!stream) return 0;
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo((hipStream_t)stream, &st, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        return 0;
+    }
+    return st == hipStreamCaptureStatusActive ? (int64_t)id + 1 : 0;
+}
+
 const char* vq2_last_error(void) { return g_err; }
 
 // The fused-rotation entries read perm / sign with vector loads.

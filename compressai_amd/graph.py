@@ -15,6 +15,8 @@ from __future__ import annotations
 
 import torch
 
+from .kernels import take_workspaces
+
 
 class DecodeStepGraph:
     """Capture ``step(*inputs)`` once and replay it for new inputs.
@@ -35,9 +37,12 @@ class DecodeStepGraph:
             for _ in range(warmup):
                 step(*self.static_in)
         cur.wait_stream(side)
+        # captured on the warm-up's stream, so that the launches take the
+        # workspaces allocated and cleared there, which become the graph's own
         self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
+        with torch.cuda.graph(self.graph, stream=side):
             self.static_out = step(*self.static_in)
+        self._workspaces = take_workspaces(side)
 
     def __call__(self, *inputs):
         if len(inputs) != len(self.static_in):

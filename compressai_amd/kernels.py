@@ -256,18 +256,31 @@ def vq_gemv(xr, i0, i1, cb0, cb1, scale, out, n, rs=1.0, *, out_dtype=torch.bflo
 # into it on every replay.
 _WS: dict = {}
 _WS_RETIRED: list = []
+# (device, stream, kind) -> (capture, workspace) of the stream's latest capture;
+# an earlier one's memory is its graph's
+_WS_CAPTURE: dict = {}
 
 
 def _workspace(dev: torch.device, nbytes: int, *, sorted_kind: bool = False) -> torch.Tensor | None:
     """The workspace of this (device, stream).  vq_sorted_gemv and
     vq_sorted_moe share one of their own, allocated zeroed: it begins with
     arrival counters that must be zero before a launch (each call leaves them
-    zero), which another kernel's partials must never overwrite."""
+    zero), which another kernel's partials must never overwrite.  A captured
+    call that finds none takes one of its graph's own: its clearing is
+    recorded and happens in that graph's replays alone, so another graph, or
+    an eager call, must not build on it."""
     if nbytes == 0:
         return None
     key = (dev.index, torch.cuda.current_stream(dev).cuda_stream, sorted_kind)
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
+        capture = _lib.load().vq2_stream_capture_id(key[1]) if sorted_kind else 0
+        if capture:
+            held = _WS_CAPTURE.get(key)
+            if held is None or held[0] != capture or held[1].numel() < nbytes:
+                held = capture, torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
+                _WS_CAPTURE[key] = held
+            return held[1]
         alloc = torch.zeros if sorted_kind else torch.empty
         new = alloc(max(nbytes, 1 << 20), dtype=torch.uint8, device=dev)
         if buf is not None:
@@ -277,6 +290,14 @@ def _workspace(dev: torch.device, nbytes: int, *, sorted_kind: bool = False) -> 
         buf = new
         _WS[key] = buf
     return buf
+
+
+def take_workspaces(stream: torch.cuda.Stream) -> list:
+    """The workspaces of `stream`, which are its no more: the caller keeps
+    them while launches that were given them may run (a graph captured on the
+    stream), and later calls there take new ones."""
+    keys = [k for k in _WS if k[0] == stream.device.index and k[1] == stream.cuda_stream]
+    return [_WS.pop(k) for k in keys]
 
 
 # The sorted workspace's header (include/vq2_amd.h): arrival counters, and in
@@ -296,7 +317,10 @@ def vq_sorted_moe_status(device=None, *, clear=False) -> int:
     dev = torch.device(device) if device is not None else torch.device("cuda", torch.cuda.current_device())
     if dev.index is None:
         dev = torch.device("cuda", torch.cuda.current_device())
-    buf = _WS.get((dev.index, torch.cuda.current_stream(dev).cuda_stream, True))
+    key = (dev.index, torch.cuda.current_stream(dev).cuda_stream, True)
+    buf = _WS.get(key)
+    if buf is None and key in _WS_CAPTURE:  # only captured calls: the latest graph's
+        buf = _WS_CAPTURE[key][1]
     if buf is None:
         return 0
     st = int(_lib.load().vq2_sorted_moe_status(buf.data_ptr(), 1 if clear else 0, _stream(dev)))

@@ -51,6 +51,10 @@ extern "C" {
 /* Library version (major*10000 + minor*100 + patch). */
 int vq2_version(void);
 
+/* A number of the capture that the stream is in, another for every capture of
+ * the process; 0 where it is in none. */
+int64_t vq2_stream_capture_id(void* stream);
+
 /* Thread-local description of the last error on this thread ("" if none). */
 const char* vq2_last_error(void);
 
@@ -394,7 +398,8 @@ int vq2_sorted_pack(const int16_t* idx0, const int16_t* idx1, int64_t out_rows, 
  * before the first call that uses the workspace (e.g. allocate it zeroed);
  * every call leaves it zero.  One workspace may serve all vq2_sorted_gemv
  * calls of a stream; calls that share a workspace must not run
- * concurrently.  A launch with several slices has at most
+ * concurrently, nor may a captured graph rely on another graph's clearing
+ * (vq2_stream_capture_id).  A launch with several slices has at most
  * VQ2_SORTED_MAX_COUNTERS chunks. */
 #define VQ2_SORTED_WS_HEADER 16384
 /* The header's last 128-byte line holds vq2_sorted_moe's status word

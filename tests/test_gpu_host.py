@@ -10,6 +10,7 @@ import pytest
 import torch
 
 from compressai_amd import _lib, kernels as K, synth
+from compressai_amd.graph import DecodeStepGraph
 from compressai_amd.kernels import Vq2Error
 from compressai_amd.moe import ResidentMoEExperts
 
@@ -149,3 +150,41 @@ def test_declined_calls(dev):
     # uint16 planes: handled by the Python entry
     (y,) = K.vq_gemv_rht(x, [(i0.view(torch.uint16), None, sc, 64)], cb0, None, n, hb=n)
     assert torch.equal(y, K.vq_gemv_rht(x, [(i0, None, sc, 64)], cb0, None, n, hb=n)[0])
+
+
+def test_every_graph_clears_the_counters_it_uses(dev):
+    """Graphs captured on one stream without an eager call before: each takes
+    a workspace of its own and clears it, so they may be replayed in any order
+    and their results are the eager ones.  A DecodeStepGraph keeps the
+    workspace its warm-up cleared, apart from its stream's later calls."""
+    n, rows = 2048, (6144, 6144)  # slices: counters of the workspace
+    ms, cb0, cb1 = _mats(dev, 8890, n, rows, 4)
+    mats = [(K.SortedPlanes(m["idx0"], m["idx1"], r, n, device=dev), m["scale"].to(dev)) for m, r in zip(ms, rows)]
+    xs = [synth.activations(8895 + i, n, dtype=torch.float16).to(dev) for i in range(3)]
+    refs = [K.vq_sorted_gemv(x, mats, cb0, cb1, n) for x in xs]
+    stream, used = torch.cuda.Stream(dev), []
+    K.take_workspaces(stream)  # (a pooled stream: an earlier user's)
+    torch.cuda.synchronize(dev)
+
+    def capture(x):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=stream):
+            for _ in range(2):
+                ys = K.vq_sorted_gemv(x, mats, cb0, cb1, n)
+            used.append(K._workspace(dev, 1 << 16, sorted_kind=True).data_ptr())
+        return g, ys
+
+    graphs = [capture(x) for x in xs]
+    assert len(set(used)) == 3
+    for i in (2, 0, 1, 2, 2, 0):
+        graphs[i][0].replay()
+        torch.cuda.synchronize(dev)
+        assert all(torch.equal(a, b) for a, b in zip(graphs[i][1], refs[i])), i
+        with torch.cuda.stream(stream):  # the stream's eager calls have their own
+            assert all(torch.equal(a, b) for a, b in zip(K.vq_sorted_gemv(xs[1], mats, cb0, cb1, n), refs[1]))
+        torch.cuda.synchronize(dev)
+    steps = [DecodeStepGraph(lambda x: K.vq_sorted_gemv(x, mats, cb0, cb1, n), [x]) for x in xs[:2]]
+    own = [w.data_ptr() for s in steps for w in s._workspaces]
+    assert len(set(own)) == len(own) >= 2 and not set(own) & {w.data_ptr() for w in K._WS.values()}
+    for i in (1, 0, 2, 1):
+        assert all(torch.equal(a, b) for a, b in zip(steps[i % 2](xs[i]), refs[i]))
